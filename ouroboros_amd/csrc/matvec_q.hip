@@ -9,7 +9,8 @@
 // payload byte with its 4 or 5 trits, so consecutive lanes read consecutive
 // payload bytes.  matmul_q decodes each byte once for up to 8 columns; a
 // 4-byte-aligned TL1 payload of several columns goes to the int8 MFMA pass of
-// tl1_mfma.hip instead (one pass over the payload for all columns).
+// tl1_mfma.hip instead (one pass over the payload for all columns), the
+// block-quantised kinds to kquant.hip and dense rows to dense_mv.hip.
 #include "common.hpp"
 
 #include <mutex>
@@ -33,6 +34,8 @@ int tl1_mfma_matmul_raw(const uint8_t *raw, size_t M, size_t K, const float *x, 
                         void *stream);
 int kq_matmul(const void *payload, int kind, size_t out_len, size_t in_len, const float *x, size_t k, float *y,
               void *stream);
+int dense_matmul(const void *payload, int kind, size_t out_len, size_t in_len, const float *x, size_t k, float *y,
+                 void *stream);
 size_t tq1_lut_partial_floats(size_t out_len, size_t in_len);
 bool tq1_lut_fits(const void *payload, size_t in_len);
 int tq1_lut_matvec(const void *payload, size_t out_len, size_t in_len, const float *x, float *y, float *partial,
@@ -164,40 +167,6 @@ __global__ __launch_bounds__(64 * kWaves) void tq1_kernel(MvArgs a) {
     wave_store<NC>(acc, a, row, c0, lane);
 }
 
-template <int KIND>
-__device__ __forceinline__ float dense_w(const uint8_t *w, long long i);
-template <>
-__device__ __forceinline__ float dense_w<OURO_KIND_F32>(const uint8_t *w, long long i) {
-    return reinterpret_cast<const float *>(w)[i];
-}
-template <>
-__device__ __forceinline__ float dense_w<OURO_KIND_F16>(const uint8_t *w, long long i) {
-    return f16_bits_to_f32(reinterpret_cast<const uint16_t *>(w)[i]);
-}
-template <>
-__device__ __forceinline__ float dense_w<OURO_KIND_BF16>(const uint8_t *w, long long i) {
-    return bf16_bits_to_f32(reinterpret_cast<const uint16_t *>(w)[i]);
-}
-
-template <int KIND, int NC>
-__global__ __launch_bounds__(64 * kWaves) void dense_kernel(MvArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * kWaves + (threadIdx.x >> 6);
-    const int c0 = blockIdx.y * NC;
-    if (row >= a.out_len) return;
-    float acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = 0.f;
-    const long long rb = static_cast<long long>(row) * a.in_len;
-    for (int i = lane; i < a.in_len; i += 64) {
-        const float w = dense_w<KIND>(a.w, rb + i);
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-            if (c0 + c < a.k) acc[c] += w * a.x[static_cast<long long>(c0 + c) * a.in_len + i];
-    }
-    wave_store<NC>(acc, a, row, c0, lane);
-}
-
 int launch_mv(int kind, const MvArgs &a, hipStream_t s) {
     const int nc = a.k >= 8 ? 8 : (a.k >= 4 ? 4 : (a.k >= 2 ? 2 : 1));
     dim3 grid((a.out_len + kWaves - 1) / kWaves, (a.k + nc - 1) / nc), block(64 * kWaves);
@@ -212,24 +181,6 @@ int launch_mv(int kind, const MvArgs &a, hipStream_t s) {
     switch (kind) {
     case OURO_KIND_TL1: OURO_MV_LAUNCH(tl1_kernel); break;
     case OURO_KIND_TQ1_0: OURO_MV_LAUNCH(tq1_kernel); break;
-    case OURO_KIND_F32:
-        if (nc == 8) hipLaunchKernelGGL((dense_kernel<OURO_KIND_F32, 8>), grid, block, 0, s, a);
-        else if (nc == 4) hipLaunchKernelGGL((dense_kernel<OURO_KIND_F32, 4>), grid, block, 0, s, a);
-        else if (nc == 2) hipLaunchKernelGGL((dense_kernel<OURO_KIND_F32, 2>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((dense_kernel<OURO_KIND_F32, 1>), grid, block, 0, s, a);
-        break;
-    case OURO_KIND_F16:
-        if (nc == 8) hipLaunchKernelGGL((dense_kernel<OURO_KIND_F16, 8>), grid, block, 0, s, a);
-        else if (nc == 4) hipLaunchKernelGGL((dense_kernel<OURO_KIND_F16, 4>), grid, block, 0, s, a);
-        else if (nc == 2) hipLaunchKernelGGL((dense_kernel<OURO_KIND_F16, 2>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((dense_kernel<OURO_KIND_F16, 1>), grid, block, 0, s, a);
-        break;
-    case OURO_KIND_BF16:
-        if (nc == 8) hipLaunchKernelGGL((dense_kernel<OURO_KIND_BF16, 8>), grid, block, 0, s, a);
-        else if (nc == 4) hipLaunchKernelGGL((dense_kernel<OURO_KIND_BF16, 4>), grid, block, 0, s, a);
-        else if (nc == 2) hipLaunchKernelGGL((dense_kernel<OURO_KIND_BF16, 2>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((dense_kernel<OURO_KIND_BF16, 1>), grid, block, 0, s, a);
-        break;
     default:
         return fail(OURO_ERR_KIND, "matvec_q: kind %d not supported", kind);
     }
@@ -265,6 +216,10 @@ int matmul_q(const void *payload, int kind, size_t out_len, size_t in_len, const
     if (out_len > 0x7fffffffULL || in_len > 0x7fffffffULL || k > 0x7fffffffULL)
         return fail(OURO_ERR_SHAPE, "matvec_q: shape too large");
     if (is_kquant(kind)) return kq_matmul(payload, kind, out_len, in_len, x, k, y, stream);
+    auto dense = [&] {
+        if ((k + 7) / 8 > 65535) return fail(OURO_ERR_SHAPE, "matmul_q: too many columns");
+        return dense_matmul(payload, kind, out_len, in_len, x, k, y, stream);
+    };
     switch (kind) {
     case OURO_KIND_TL1:
         if (in_len % 128) return fail(OURO_ERR_SHAPE, "matvec_q TL1: in_len %zu not a multiple of 128", in_len);
@@ -298,11 +253,11 @@ int matmul_q(const void *payload, int kind, size_t out_len, size_t in_len, const
         break;
     case OURO_KIND_F32:
         if (reinterpret_cast<uintptr_t>(payload) % 4) return fail(OURO_ERR_ALIGN, "matvec_q F32: payload alignment");
-        break;
+        return dense();
     case OURO_KIND_F16:
     case OURO_KIND_BF16:
         if (reinterpret_cast<uintptr_t>(payload) % 2) return fail(OURO_ERR_ALIGN, "matvec_q F16: payload alignment");
-        break;
+        return dense();
     case OURO_KIND_I2:
     case OURO_KIND_I2_S: {
         const size_t tb = i2_tiled_bytes(out_len, in_len);
