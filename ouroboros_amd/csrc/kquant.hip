@@ -23,6 +23,11 @@
 // the whole launch), so the per-element work is a share of a mask and three
 // quarter-width dot steps.
 //
+// Several columns (matmul_q) are taken up to four at a time by every kernel
+// here: the codes are read and decoded once for the group, and each column's
+// products, scales and sums are those of a single column, so a column of
+// matmul_q is matvec_q of it bit for bit (kq_columns).
+//
 // Mapping.  A thread owns one task position of a row (k-stationary): its 32 x
 // values and their run sums stay in registers while the workgroup walks row
 // tiles, so x is read once per workgroup.  A workgroup is `slots` side-by-side
@@ -54,6 +59,7 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxThreads = 1024;
 
@@ -135,17 +141,21 @@ __device__ __forceinline__ void make_run(const float *p, XRun &r) {
     (void)frexpf(m, &E);  // m = f 2^E, f in [0.5, 1): |x| < 2^E (E = 0 for m = 0)
     // a non-finite x makes the run's sum NaN
     r.s = __builtin_isfinite(m) ? ldexpf(1.0f, E - 22) : __builtin_nanf("");
-    uint32_t w0[4] = {0, 0, 0, 0}, w1[4] = {0, 0, 0, 0}, w2[4] = {0, 0, 0, 0};
+    // x_int + 0x808080 has the balanced digits plus 128 as its bytes; a xor
+    // takes the 128s off, and byte permutes gather the planes of four elements
+    uint32_t w0[4], w1[4], w2[4];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int xi = __builtin_isfinite(m) ? static_cast<int>(rintf(ldexpf(v[i], 22 - E))) : 0;
-        const int p2 = ((xi + 128) & 255) - 128;
-        const int r1 = (xi - p2) >> 8;  // exact: xi - p2 is a multiple of 256
-        const int p1 = ((r1 + 128) & 255) - 128;
-        const int p0 = (r1 - p1) >> 8;
-        w0[i >> 2] |= static_cast<uint32_t>(p0 & 255) << (8 * (i & 3));
-        w1[i >> 2] |= static_cast<uint32_t>(p1 & 255) << (8 * (i & 3));
-        w2[i >> 2] |= static_cast<uint32_t>(p2 & 255) << (8 * (i & 3));
+    for (int d = 0; d < 4; ++d) {
+        uint32_t t[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int xi = __builtin_isfinite(m) ? static_cast<int>(rintf(ldexpf(v[4 * d + i], 22 - E))) : 0;
+            t[i] = (static_cast<uint32_t>(xi) + 0x808080u) ^ 0x808080u;
+        }
+        const uint32_t a = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), b = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
+        w2[d] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+        w1[d] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        w0[d] = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0602u) | __builtin_amdgcn_perm(t[3], t[2], 0x06020c0cu);
     }
     r.p0 = u32x4{w0[0], w0[1], w0[2], w0[3]};
     r.p1 = u32x4{w1[0], w1[1], w1[2], w1[3]};
@@ -198,9 +208,11 @@ template <> struct Fmt<OURO_KIND_Q8_0> {
         r.d1 = bp[1];
         return r;
     }
-    __device__ static float dot(const Raw &r, int, const XRun &xa, const XRun &xb) {
+    template <int NC>
+    __device__ static void dots(const Raw &r, int, const XRun (&xa)[NC], const XRun (&xb)[NC], float (&v)[NC]) {
         const float d = f16f(r.d0 | (r.d1 << 8));
-        return d * (idot(r.a, xa) + idot(r.b, xb));
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] = d * (idot(r.a, xa[c]) + idot(r.b, xb[c]));
     }
 };
 
@@ -230,17 +242,22 @@ template <> struct Fmt<OURO_KIND_Q4K> {
     template <bool AL16, bool PH> __device__ static Raw load(const uint8_t *bp, int u, const uint32_t *sh) {
         return Raw{piece<AL16, PH>(bp, 0, sh, 0), piece<AL16, PH>(bp, 16 + 16 * u, sh, 1)};
     }
-    __device__ static float dot(const Raw &r, int u, const XRun &xa, const XRun &xb) {
+    template <int NC>
+    __device__ static void dots(const Raw &r, int u, const XRun (&xa)[NC], const XRun (&xb)[NC], float (&v)[NC]) {
 #pragma clang fp contract(off)
         const int j = u >> 1;
         uint32_t s1, m1, s2, m2;
         scale_min_k4(2 * j, r.h.y, r.h.z, r.h.w, s1, m1);
         scale_min_k4(2 * j + 1, r.h.y, r.h.z, r.h.w, s2, m2);
         const float d = f16f(r.h.x & 0xffffu), dmin = f16f(r.h.x >> 16);
-        const float SA = idot(vmap(r.q, 0x0f0f0f0fu, 0), xa);
-        const float SB = idot(vmap(r.q, 0x0f0f0f0fu, 4), xb);
-        return (d * static_cast<float>(s1)) * SA - (dmin * static_cast<float>(m1)) * xa.X +
-               ((d * static_cast<float>(s2)) * SB - (dmin * static_cast<float>(m2)) * xb.X);
+        const u32x4 lo = vmap(r.q, 0x0f0f0f0fu, 0), hi = vmap(r.q, 0x0f0f0f0fu, 4);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const float SA = idot(lo, xa[c]);
+            const float SB = idot(hi, xb[c]);
+            v[c] = (d * static_cast<float>(s1)) * SA - (dmin * static_cast<float>(m1)) * xa[c].X +
+                   ((d * static_cast<float>(s2)) * SB - (dmin * static_cast<float>(m2)) * xb[c].X);
+        }
     }
 };
 
@@ -255,7 +272,8 @@ template <> struct Fmt<OURO_KIND_Q5K> {
         return Raw{piece<AL16, PH>(bp, 0, sh, 0), piece<AL16, PH>(bp, 16 + 16 * (u & 1), sh, 1),
                    piece<AL16, PH>(bp, 48 + 16 * u, sh, 2)};
     }
-    __device__ static float dot(const Raw &r, int u, const XRun &xa, const XRun &xb) {
+    template <int NC>
+    __device__ static void dots(const Raw &r, int u, const XRun (&xa)[NC], const XRun (&xb)[NC], float (&v)[NC]) {
 #pragma clang fp contract(off)
         const int j = u >> 1;
         uint32_t s1, m1, s2, m2;
@@ -265,10 +283,13 @@ template <> struct Fmt<OURO_KIND_Q5K> {
         // bit 2j / 2j + 1 of qh to bit 4 of each byte
         const u32x4 lo = merge_hi(r.q, 0x0f0f0f0fu, r.qh, 2 * j - 4, 0x10101010u);
         const u32x4 hi = merge_hi(vmap(r.q, 0xffffffffu, 4), 0x0f0f0f0fu, r.qh, 2 * j - 3, 0x10101010u);
-        const float SA = idot(lo, xa);
-        const float SB = idot(hi, xb);
-        return (d * static_cast<float>(s1)) * SA - (dmin * static_cast<float>(m1)) * xa.X +
-               ((d * static_cast<float>(s2)) * SB - (dmin * static_cast<float>(m2)) * xb.X);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const float SA = idot(lo, xa[c]);
+            const float SB = idot(hi, xb[c]);
+            v[c] = (d * static_cast<float>(s1)) * SA - (dmin * static_cast<float>(m1)) * xa[c].X +
+                   ((d * static_cast<float>(s2)) * SB - (dmin * static_cast<float>(m2)) * xb[c].X);
+        }
     }
 };
 
@@ -297,18 +318,22 @@ template <> struct Fmt<OURO_KIND_Q6K> {
         r.d1 = bp[209];
         return r;
     }
-    __device__ static float dot(const Raw &r, int u, const XRun &xa, const XRun &xb) {
+    template <int NC>
+    __device__ static void dots(const Raw &r, int u, const XRun (&xa)[NC], const XRun (&xb)[NC], float (&v)[NC]) {
 #pragma clang fp contract(off)
         const int s = u & 1;
         const float d = f16f(r.d0 | (r.d1 << 8));
         // bits 2s, 2s + 1 / 4 + 2s, 5 + 2s of qh to bits 4, 5 of each byte
         const u32x4 lo = merge_hi(r.ql, 0x0f0f0f0fu, r.qh, 2 * s - 4, 0x30303030u);
         const u32x4 hi = merge_hi(vmap(r.ql, 0xffffffffu, 4), 0x0f0f0f0fu, r.qh, 2 * s, 0x30303030u);
-        const float SA = idot(lo, xa) - 32.f * xa.X;
-        const float SB = idot(hi, xb) - 32.f * xb.X;
         const float ca = d * static_cast<float>(static_cast<int8_t>(r.sa));
         const float cb = d * static_cast<float>(static_cast<int8_t>(r.sb));
-        return ca * SA + cb * SB;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const float SA = idot(lo, xa[c]) - 32.f * xa[c].X;
+            const float SB = idot(hi, xb[c]) - 32.f * xb[c].X;
+            v[c] = ca * SA + cb * SB;
+        }
     }
 };
 
@@ -341,7 +366,8 @@ template <> struct Fmt<OURO_KIND_Q3K> {
         r.d1 = bp[109];
         return r;
     }
-    __device__ static float dot(const Raw &r, int u, const XRun &xa, const XRun &xb) {
+    template <int NC>
+    __device__ static void dots(const Raw &r, int u, const XRun (&xa)[NC], const XRun (&xb)[NC], float (&v)[NC]) {
 #pragma clang fp contract(off)
         const int n = u >> 2, t = u & 1, l0 = 16 * ((u >> 1) & 1);
         const int ka = 8 * n + 4 * t + (l0 >> 4), kb = ka + 2;
@@ -355,11 +381,14 @@ template <> struct Fmt<OURO_KIND_Q3K> {
         const u32x4 qs = vmap(r.q, 0xffffffffu, 2 * j0);
         const u32x4 ca = merge_hi(qs, 0x03030303u, r.hm, 4 * n + j0 - 2, 0x04040404u);
         const u32x4 cb = merge_hi(qs, 0x0c0c0c0cu, r.hm, 4 * n + j0 - 3, 0x10101010u);
-        const float SA = idot(ca, xa) - 4.f * xa.X;
-        const float SB = 0.25f * idot(cb, xb) - 4.f * xb.X;
         const float fa = d * (static_cast<float>(sa) - 32.f);
         const float fb = d * (static_cast<float>(sb) - 32.f);
-        return fa * SA + fb * SB;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const float SA = idot(ca, xa[c]) - 4.f * xa[c].X;
+            const float SB = 0.25f * idot(cb, xb[c]) - 4.f * xb[c].X;
+            v[c] = fa * SA + fb * SB;
+        }
     }
 };
 
@@ -372,6 +401,7 @@ struct KqArgs {
     int tpr;    // tasks per row
     int slots;  // row task sets side by side in a workgroup
     int tiles;  // ceil(out_len / (slots * R))
+    int k;
 };
 // passed by value to a kernel: the host and device passes must lay it out
 // alike (56 bytes in the code object's kernel-argument metadata)
@@ -394,7 +424,7 @@ __device__ __forceinline__ void load_x(const float *xc, int blk, int u, XRun &xa
 // Several task sets per workgroup (slots > 1): each thread's sum of each row
 // of a batch of up to kBatch tiles, red[(b R + r) nt + t]; one wavefront per
 // row adds a row's task sums.
-constexpr int kBatch = 4;
+constexpr int kBatch = 4;  // tiles times columns
 // One task set per workgroup (slots == 1): each wavefront adds its lanes'
 // sums in registers and keeps one value per row, red[(b R + r) nwaves +
 // wave], for a batch of up to kBatch1 tiles.
@@ -407,29 +437,29 @@ constexpr int kBatch1 = 64;
 __device__ __forceinline__ void vm_drain() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
 template <int R>
-__device__ __forceinline__ void stash(float *red, const float (&v)[R], int b) {
+__device__ __forceinline__ void stash(float *red, const float (&v)[R], int b) {  // b: tile of the batch, column by column
     const int t = threadIdx.x, nt = blockDim.x;
 #pragma unroll
     for (int r = 0; r < R; ++r) red[(b * R + r) * nt + t] = v[r];
 }
 
 // Rows of the nb tiles tile0, tile0 + g, ... of a batch.
-template <int R>
-__device__ __forceinline__ void flush(const KqArgs &a, const float *red, int nb, int tile0, int g, int col) {
+template <int R, int NC>
+__device__ __forceinline__ void flush(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0) {
     const int t = threadIdx.x, nt = blockDim.x;
     const int rows_per_tile = a.slots * R;
     const int wave = t >> 6, lane = t & 63, nwaves = nt >> 6;
     __syncthreads();
-    for (int o = wave; o < nb * rows_per_tile; o += nwaves) {
-        const int b = o / rows_per_tile, ob = o - b * rows_per_tile;
+    for (int o = wave; o < nb * NC * rows_per_tile; o += nwaves) {
+        const int b = o / rows_per_tile, ob = o - b * rows_per_tile, col = c0 + b % NC;
         const int s = ob / R, r = ob - s * R;
         const float *src = red + (b * R + r) * nt + s * a.tpr;
         float acc = 0.f;
         for (int i = lane; i < a.tpr; i += 64) acc += src[i];
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) acc += xor_shfl(acc, off);
-        const int row = (tile0 + b * g) * rows_per_tile + ob;
-        if (lane == 0 && row < a.out_len) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
+        const int row = (tile0 + b / NC * g) * rows_per_tile + ob;
+        if (lane == 0 && row < a.out_len && col < a.k) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
     }
     __syncthreads();
     vm_drain();
@@ -490,16 +520,16 @@ __device__ __forceinline__ void stash1(float *red, float (&v)[R], int b, bool li
     if (lane % span == span - 1) red[(b * R + lane / span) * nwaves + wave] = s;
 }
 
-template <int R>
-__device__ __forceinline__ void flush1(const KqArgs &a, const float *red, int nb, int tile0, int g, int col) {
+template <int R, int NC>
+__device__ __forceinline__ void flush1(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0) {
     const int t = threadIdx.x, nwaves = blockDim.x >> 6;
     __syncthreads();
-    for (int o = t; o < nb * R; o += blockDim.x) {
-        const int b = o / R, r = o - b * R;
+    for (int o = t; o < nb * NC * R; o += blockDim.x) {
+        const int b = o / R, r = o - b * R, col = c0 + b % NC;
         float acc = 0.f;
         for (int w = 0; w < nwaves; ++w) acc += red[(b * R + r) * nwaves + w];
-        const int row = (tile0 + b * g) * R + r;
-        if (row < a.out_len) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
+        const int row = (tile0 + b / NC * g) * R + r;
+        if (row < a.out_len && col < a.k) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
     }
     __syncthreads();
     vm_drain();
@@ -513,10 +543,10 @@ __device__ __forceinline__ void flush1(const KqArgs &a, const float *red, int nb
 // (136 -> 128 VGPRs, no spill); the other kinds are left as the compiler
 // allocates them (4 waves already; Q8_0 held to 5 ran 10 % slower, the
 // others spill when pressed).
-template <int KIND> constexpr int kWavesPerSimd = KIND == OURO_KIND_Q3K ? 4 : 1;
+template <int KIND, int NC> constexpr int kWavesPerSimd = KIND == OURO_KIND_Q3K && NC == 1 ? 4 : 1;
 
-template <int KIND, int R, bool AL16, bool PH, int MAXT>
-__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<KIND>)))
+template <int KIND, int R, bool AL16, bool PH, int MAXT, int NC>
+__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<KIND, NC>)))
 void kq_gemv_kernel(KqArgs a) {
     using F = Fmt<KIND>;
     extern __shared__ float red[];  // slots == 1: [kBatch1][R][wavefronts], else [kBatch][R][blockDim.x]
@@ -524,9 +554,11 @@ void kq_gemv_kernel(KqArgs a) {
     const int slot = min(t / a.tpr, a.slots - 1);
     const int task = min(t - slot * a.tpr, a.tpr - 1);
     const int blk = task / F::TPB, u = task % F::TPB;
-    const int col = blockIdx.y;
-    XRun xa, xb;
-    load_x<KIND>(a.x + static_cast<long long>(col) * a.in_len, blk, u, xa, xb);
+    const int c0 = blockIdx.y * NC;
+    XRun xa[NC], xb[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)  // clamped columns are dropped
+        load_x<KIND>(a.x + static_cast<long long>(min(c0 + c, a.k - 1)) * a.in_len, blk, u, xa[c], xb[c]);
     const int rows_per_tile = a.slots * R;
     const uint8_t *wb = a.w + static_cast<long long>(blk) * F::BB;
     // a row is under 4 GiB (the host checks), so its offset is one 32 x 32 -> 64-bit multiply-add
@@ -550,18 +582,27 @@ void kq_gemv_kernel(KqArgs a) {
     // sum one tile into the batch; a full batch, or the last tile, is added up
     const bool one = a.slots == 1;          // uniform
     const bool live = t < a.tpr * a.slots;  // not a padding lane
-    const int batch = one ? kBatch1 : kBatch;
+    constexpr int kB1 = kBatch1 / NC, kB = kBatch / NC;
+    const int batch = one ? kB1 : kB;
     auto sum = [&](const typename F::Raw(&raw)[R]) {
-        float v[R];
+        float v[NC][R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = F::dot(raw[r], u, xa, xb);
-        if (one) stash1<R>(red, v, nb, live);
-        else stash<R>(red, v, nb);
+        for (int r = 0; r < R; ++r) {
+            float vc[NC];
+            F::template dots<NC>(raw[r], u, xa, xb, vc);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) v[c][r] = vc[c];
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (one) stash1<R>(red, v[c], nb * NC + c, live);
+            else stash<R>(red, v[c], nb * NC + c);
+        }
         ++nb;
         tile += g;
         if (nb == batch || tile >= a.tiles) {  // uniform over the workgroup
-            if (one) flush1<R>(a, red, nb, tile0, g, col);
-            else flush<R>(a, red, nb, tile0, g, col);
+            if (one) flush1<R, NC>(a, red, nb, tile0, g, c0);
+            else flush<R, NC>(a, red, nb, tile0, g, c0);
             nb = 0;
             tile0 = tile;
         }
@@ -597,12 +638,14 @@ __global__ __launch_bounds__(256) void kq_row_kernel(KqArgs a) {
     float acc = 0.f;
     for (int task = lane; task < a.tpr; task += 64) {
         const int blk = task / F::TPB, u = task % F::TPB;
-        XRun xa, xb;
-        load_x<KIND>(xc, blk, u, xa, xb);
+        XRun xa[1], xb[1];
+        load_x<KIND>(xc, blk, u, xa[0], xb[0]);
         const uint32_t none[F::NP] = {};
         const typename F::Raw raw =
             F::template load<false, false>(a.w + row * a.row_bytes + static_cast<long long>(blk) * F::BB, u, none);
-        acc += F::dot(raw, u, xa, xb);
+        float v[1];
+        F::template dots<1>(raw, u, xa, xb, v);
+        acc += v[0];
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) acc += xor_shfl(acc, off);
@@ -706,9 +749,9 @@ __device__ __forceinline__ u32x4 q3_flip(u32x4 P) {
 // One block of the lane's row: the four runs' MFMAs, then d.  aoff: the
 // lane's A slot within a run's planes; hr[j]: the rotation that brings
 // hmask bit 4n + j to bit 7.
-template <int PAR>
-__device__ __forceinline__ float q3_block(const Q3Raw &r, const uint8_t *xlds, int b, int aoff,
-                                          const uint32_t (&hr)[4], uint32_t L, int g) {
+template <int PAR, int NC>
+__device__ __forceinline__ void q3_block(const Q3Raw &r, const uint8_t *xlds, int b, int nb, int aoff,
+                                         const uint32_t (&hr)[4], uint32_t L, int g, float (&out)[NC]) {
 #pragma clang fp contract(off)
     constexpr int PO = kQ3PO<PAR>;
     u32x4 q = r.q, h = r.h;
@@ -718,37 +761,46 @@ __device__ __forceinline__ float q3_block(const Q3Raw &r, const uint8_t *xlds, i
     }
     const u32x4 hn = ~h;
     const u32x4 P = q3_flip<PO>(r.P);
-    const uint8_t *xb = xlds + b * kQ3Unit;
-    const float4 xs = *reinterpret_cast<const float4 *>(xb + 4 * kQ3Run + 16 * g);
-    float blk = 0.f;
+    const uint8_t *xb = xlds + b * kQ3Unit;  // column i: nb units further each
+    f32x4 xs[NC];
+    float blk[NC] = {};
+#pragma unroll
+    for (int i = 0; i < NC; ++i) xs[i] = *reinterpret_cast<const f32x4 *>(xb + i * nb * kQ3Unit + 4 * kQ3Run + 16 * g);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + kQ3Run * j + aoff);
         q3v4i B;
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
             const uint32_t qv = __builtin_amdgcn_alignbit(q[d], q[d], (2 * j - 5) & 31) & 0x60606060u;
             B[d] = static_cast<int>(qv | (__builtin_amdgcn_alignbit(hn[d], hn[d], hr[j]) & 0x80808080u));
         }
-        const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B, q3v4i{0, 0, 0, 0}, 0, 0, 0);
-        const int t = (D[1] << 3) + (D[2] >> 5);
-        const int U = (D[0] << 11) + t;
         int s;
         if (j == 0) s = q3_scale<PO, 0>(P, L);
         else if (j == 1) s = q3_scale<PO, 1>(P, L);
         else if (j == 2) s = q3_scale<PO, 2>(P, L);
         else s = q3_scale<PO, 3>(P, L);
-        const float xsj = j == 0 ? xs.x : j == 1 ? xs.y : j == 2 ? xs.z : xs.w;
-        blk = __builtin_fmaf(static_cast<float>(s), xsj * static_cast<float>(U), blk);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + i * nb * kQ3Unit + kQ3Run * j + aoff);
+            const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B, q3v4i{0, 0, 0, 0}, 0, 0, 0);
+            const int t = (D[1] << 3) + (D[2] >> 5);
+            const int U = (D[0] << 11) + t;
+            blk[i] = __builtin_fmaf(static_cast<float>(s), xs[i][j] * static_cast<float>(U), blk[i]);
+        }
     }
     const uint32_t dbits = PAR == 0 ? (r.P.w & 0xffffu) : (r.P.w >> 16);
-    return f16f(dbits) * blk;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) out[i] = f16f(dbits) * blk[i];
 }
 
 // x's digit planes of every run into LDS; rot_odd: the element order of the
 // odd blocks' B slices (2: elements 2, .., 15, 0, 1).
-__device__ __forceinline__ void q3_prep(const float *xc, int nb, uint8_t *xlds, int rot_odd) {
-    for (int run = threadIdx.x; run < nb * 16; run += blockDim.x) {
+// (columns c0 .. c0 + NC - 1, each nb units after the other; clamped ones are dropped)
+template <int NC>
+__device__ __forceinline__ void q3_prep(const KqArgs &a, int c0, int nb, uint8_t *xlds, int rot_odd) {
+    for (int id = threadIdx.x; id < nb * 16 * NC; id += blockDim.x) {
+        const int cc = NC == 1 ? 0 : id / (nb * 16), run = id - cc * (nb * 16);
+        const float *xc = a.x + static_cast<long long>(min(c0 + cc, a.k - 1)) * a.in_len;
         const int b = run >> 4, g = (run >> 2) & 3, j = run & 3;
         const float *src = xc + 256 * b + 128 * (g >> 1) + 32 * j + 16 * (g & 1);
         const int rot = (b & 1) ? rot_odd : 0;
@@ -757,7 +809,7 @@ __device__ __forceinline__ void q3_prep(const float *xc, int nb, uint8_t *xlds, 
         for (int i = 0; i < 16; ++i) v[i] = src[(i + rot) & 15];
         XRun xr;
         make_run(v, xr);
-        uint8_t *xb = xlds + b * kQ3Unit;
+        uint8_t *xb = xlds + (cc * nb + b) * kQ3Unit;
         u32x4 *dst = reinterpret_cast<u32x4 *>(xb + kQ3Run * j + 48 * g);
         dst[0] = xr.p0;
         dst[1] = xr.p1;
@@ -767,14 +819,66 @@ __device__ __forceinline__ void q3_prep(const float *xc, int nb, uint8_t *xlds, 
     }
 }
 
-template <int MODE>
+// A tile's row sums: lane 16 g + c's sums of row c over the four pieces, by
+// two lane swaps.
+__device__ __forceinline__ float piece_sum(float acc) {
+    const auto q1 = __builtin_amdgcn_permlane32_swap(ubits(acc), ubits(acc), false, false);
+    acc = fbits(q1[0]) + fbits(q1[1]);
+    const auto q2 = __builtin_amdgcn_permlane16_swap(ubits(acc), ubits(acc), false, false);
+    return fbits(q2[0]) + fbits(q2[1]);
+}
+
+// Shared 16-row tiles: the wavefronts' sums of NC columns meet in LDS, every
+// wavefront once a tile (par: the tile's parity); wavefront i adds and stores
+// the columns i, i + 4, ..
+template <int NC>
+__device__ __forceinline__ void finish_sh(const KqArgs &a, float (*red)[4][16], int par, float (&acc)[NC], int tile, int c0,
+                                          int wave, int lane) {
+    const int c = lane & 15;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const float v = piece_sum(acc[i]);
+        if (lane < 16) red[par * NC + i][wave][c] = v;
+    }
+    __syncthreads();
+    const int row = tile * 16 + c;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const float(*rr)[16] = red[par * NC + i];
+        if (wave == i % 4 && lane < 16 && row < a.out_len && c0 + i < a.k)
+            a.y[static_cast<long long>(c0 + i) * a.out_len + row] = ((rr[0][c] + rr[1][c]) + rr[2][c]) + rr[3][c];
+    }
+}
+
+// 64-row tiles: each wavefront stores its 16 rows (row: the lane's).
+template <int NC>
+__device__ __forceinline__ void finish_own(const KqArgs &a, float (&acc)[NC], int row, int c0, int lane) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const float v = piece_sum(acc[i]);
+        if (lane < 16 && row < a.out_len && c0 + i < a.k) a.y[static_cast<long long>(c0 + i) * a.out_len + row] = v;
+    }
+}
+
+template <int NC>
+__device__ __forceinline__ void add(float (&acc)[NC], const float (&v)[NC]) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) acc[i] += v[i];
+}
+
+template <int NC>
+__device__ __forceinline__ void zero(float (&acc)[NC]) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) acc[i] = 0.f;
+}
+
+template <int MODE, int NC>
 __global__ __launch_bounds__(kQ3Threads) void kq3_mfma_kernel(KqArgs a) {
     constexpr bool SH = MODE == Q3K_STS;
     constexpr int RT = SH ? 16 : kQ3Rows;  // rows a tile
     extern __shared__ __attribute__((aligned(16))) uint8_t xlds[];
     const int nb = a.in_len / 256;
-    const int col = blockIdx.y;
-    const float *xc = a.x + static_cast<long long>(col) * a.in_len;
+    const int c0 = blockIdx.y * NC;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4, n = g >> 1;
     // A slot: row c = 4 g' + p holds plane p of run (g', j) in k-slot group
@@ -793,26 +897,14 @@ __global__ __launch_bounds__(kQ3Threads) void kq3_mfma_kernel(KqArgs a) {
         const int row = min(min(t, tiles - 1) * RT + rw + c, a.out_len - 1);  // clamped rows are dropped
         return a.w + static_cast<uint64_t>(static_cast<uint32_t>(row)) * rb32;
     };
-    // a row's partial sums over the four pieces, added by two lane swaps;
-    // lanes 0..15 store
-    auto finish = [&](float acc, int t) {
-        auto q1 = __builtin_amdgcn_permlane32_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q1[0]) + fbits(q1[1]);
-        auto q2 = __builtin_amdgcn_permlane16_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q2[0]) + fbits(q2[1]);
-        if constexpr (SH) {  // every wavefront, once a tile
-            float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + nb * kQ3Unit + kQ3Waves * kQ3Stage);
-            const int par = (t / static_cast<int>(gridDim.x)) & 1;
-            if (g == 0) red[par][wave][c] = acc;
-            __syncthreads();
-            const int row = t * RT + c;
-            if (wave == 0 && g == 0 && row < a.out_len)
-                a.y[static_cast<long long>(col) * a.out_len + row] =
-                    ((red[par][0][c] + red[par][1][c]) + red[par][2][c]) + red[par][3][c];
+    auto finish = [&](float (&acc)[NC], int t) {
+        if constexpr (SH) {
+            float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + NC * nb * kQ3Unit + kQ3Waves * kQ3Stage);
+            finish_sh<NC>(a, red, (t / static_cast<int>(gridDim.x)) & 1, acc, t, c0, wave, lane);
         } else {
-            const int row = t * RT + rw + c;
-            if (g == 0 && row < a.out_len) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
+            finish_own<NC>(a, acc, t * RT + rw + c, c0, lane);
         }
+        zero(acc);
     };
     const int g8 = gridDim.x;
     if constexpr (MODE != Q3K_ANY) {
@@ -822,7 +914,7 @@ __global__ __launch_bounds__(kQ3Threads) void kq3_mfma_kernel(KqArgs a) {
         // 204 (overlapping unit 12, so no read passes the segment) and stored
         // at 208, so segment bytes from 208 on sit 4 bytes later in LDS.
         const int steps = nb / 2;
-        uint8_t *wl = xlds + nb * kQ3Unit + wave * kQ3Stage;
+        uint8_t *wl = xlds + NC * nb * kQ3Unit + wave * kQ3Stage;
         int urow[4], uoff[4], ulds[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -852,13 +944,13 @@ __global__ __launch_bounds__(kQ3Threads) void kq3_mfma_kernel(KqArgs a) {
         const int s0 = SH ? wave : 0, ss = SH ? 4 : 1;
         const bool any = !SH || s0 < steps;
         int s = s0;
-        float acc = 0.f;
+        float acc[NC] = {};
         if (any) issue(tile, s0);
-        q3_prep(xc, nb, xlds, 2);  // the first loads are in flight meanwhile
+        q3_prep<NC>(a, c0, nb, xlds, 2);  // the first loads are in flight meanwhile
         __syncthreads();
         for (;;) {
             if (!any) {  // STS only
-                finish(0.f, tile);
+                finish(acc, tile);
                 tile += g8;
                 if (tile >= tiles) break;
                 continue;
@@ -883,11 +975,13 @@ __global__ __launch_bounds__(kQ3Threads) void kq3_mfma_kernel(KqArgs a) {
             const uint2 zw = *reinterpret_cast<const uint2 *>(rl + 216);
             o.P.z = zw.x;
             o.P.w = zw.y;
-            acc += q3_block<0>(e, xlds, 2 * s, aoff, hr, L, g);
-            acc += q3_block<1>(o, xlds, 2 * s + 1, aoff, hr, L, g);
+            float v[NC];
+            q3_block<0, NC>(e, xlds, 2 * s, nb, aoff, hr, L, g, v);
+            add(acc, v);
+            q3_block<1, NC>(o, xlds, 2 * s + 1, nb, aoff, hr, L, g, v);
+            add(acc, v);
             if (last) {
                 finish(acc, tile);
-                acc = 0.f;
                 s = s0;
                 tile += g8;
             } else {
@@ -899,15 +993,16 @@ __global__ __launch_bounds__(kQ3Threads) void kq3_mfma_kernel(KqArgs a) {
         Q3Raw r0, r1;
         auto issue = [&](Q3Raw &r, int t, int b) { q3_load_any(r, row_ptr(t) + 110 * b, g); };
         int b = 0;
-        float acc = 0.f;
+        float acc[NC] = {};
         issue(r0, tile, 0);
-        q3_prep(xc, nb, xlds, 0);
+        q3_prep<NC>(a, c0, nb, xlds, 0);
         __syncthreads();
         auto step = [&](const Q3Raw &r) {
-            acc += q3_block<2>(r, xlds, b, aoff, hr, L, g);
+            float v[NC];
+            q3_block<2, NC>(r, xlds, b, nb, aoff, hr, L, g, v);
+            add(acc, v);
             if (++b == nb) {
                 finish(acc, tile);
-                acc = 0.f;
                 b = 0;
                 tile += g8;
             }
@@ -947,12 +1042,15 @@ __global__ __launch_bounds__(kQ3Threads) void kq3_mfma_kernel(KqArgs a) {
 constexpr int kQ45Unit = 4 * kQ3Run + 128;  // a block's planes, then the exponents and the x sums [g][j]
 
 // x's digit planes, exponents and sums of every run (elements 256 b + 64 g + 16 j ..)
-__device__ __forceinline__ void q45_prep(const float *xc, int nb, uint8_t *xlds) {
-    for (int run = threadIdx.x; run < nb * 16; run += blockDim.x) {
+template <int NC>
+__device__ __forceinline__ void q45_prep(const KqArgs &a, int c0, int nb, uint8_t *xlds) {
+    for (int id = threadIdx.x; id < nb * 16 * NC; id += blockDim.x) {
+        const int cc = NC == 1 ? 0 : id / (nb * 16), run = id - cc * (nb * 16);
+        const float *xc = a.x + static_cast<long long>(min(c0 + cc, a.k - 1)) * a.in_len;
         const int b = run >> 4, g = (run >> 2) & 3, j = run & 3;
         XRun xr;
         make_run(xc + 256 * b + 64 * g + 16 * j, xr);
-        uint8_t *xb = xlds + b * kQ45Unit;
+        uint8_t *xb = xlds + (cc * nb + b) * kQ45Unit;
         u32x4 *dst = reinterpret_cast<u32x4 *>(xb + kQ3Run * j + 48 * g);
         dst[0] = xr.p0;
         dst[1] = xr.p1;
@@ -963,7 +1061,7 @@ __device__ __forceinline__ void q45_prep(const float *xc, int nb, uint8_t *xlds)
     }
 }
 
-template <int KIND, bool SH>
+template <int KIND, bool SH, int NC>
 __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
 #pragma clang fp contract(off)
     constexpr bool Q5 = KIND == OURO_KIND_Q5K;
@@ -972,8 +1070,7 @@ __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
     constexpr int kUnits = 16 * NU, kIns = (kUnits + 63) / 64;
     extern __shared__ __attribute__((aligned(16))) uint8_t xlds[];
     const int nb = a.in_len / 256;
-    const int col = blockIdx.y;
-    const float *xc = a.x + static_cast<long long>(col) * a.in_len;
+    const int c0 = blockIdx.y * NC;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
     const int aoff = (c >> 2) == g && (c & 3) < 3 ? 48 * g + 16 * (c & 3) : 192;
@@ -983,9 +1080,9 @@ __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
     if (tile >= tiles) return;  // the whole workgroup (blockIdx.x is uniform)
     const uint32_t rb32 = static_cast<uint32_t>(a.row_bytes);
     const int g8 = gridDim.x;
-    uint8_t *wl = xlds + nb * kQ45Unit + wave * (16 * BB);
-    // SH: the wavefronts' row sums [tile parity][wavefront][row], after the staging areas
-    float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + nb * kQ45Unit + 4 * 16 * BB);
+    uint8_t *wl = xlds + NC * nb * kQ45Unit + wave * (16 * BB);
+    // SH: the wavefronts' row sums [tile parity, column][wavefront][row], after the staging areas
+    float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + NC * nb * kQ45Unit + 4 * 16 * BB);
     int urow[kIns], uoff[kIns];
 #pragma unroll
     for (int i = 0; i < kIns; ++i) {
@@ -1008,23 +1105,10 @@ __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
         for (int i = 0; i < kIns; ++i)
             if (64 * i + lane < kUnits) *reinterpret_cast<u32x4 *>(wl + BB * urow[i] + uoff[i]) = st[i];
     };
-    auto finish = [&](float acc, int t) {
-        auto q1 = __builtin_amdgcn_permlane32_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q1[0]) + fbits(q1[1]);
-        auto q2 = __builtin_amdgcn_permlane16_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q2[0]) + fbits(q2[1]);
-        if constexpr (SH) {  // every wavefront, once a tile
-            const int par = (t / g8) & 1;
-            if (g == 0) red[par][wave][c] = acc;
-            __syncthreads();
-            const int row = t * RT + c;
-            if (wave == 0 && g == 0 && row < a.out_len)
-                a.y[static_cast<long long>(col) * a.out_len + row] =
-                    ((red[par][0][c] + red[par][1][c]) + red[par][2][c]) + red[par][3][c];
-        } else {
-            const int row = t * RT + rw + c;
-            if (g == 0 && row < a.out_len) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
-        }
+    auto finish = [&](float (&acc)[NC], int t) {
+        if constexpr (SH) finish_sh<NC>(a, red, (t / g8) & 1, acc, t, c0, wave, lane);
+        else finish_own<NC>(a, acc, t * RT + rw + c, c0, lane);
+        zero(acc);
     };
     const uint8_t *rl = wl + BB * c;
     // the wavefront's blocks of a tile: b0, b0 + bs, .. (SH: wavefronts with
@@ -1032,13 +1116,13 @@ __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
     const int b0 = SH ? wave : 0, bs = SH ? 4 : 1;
     const bool any = !SH || b0 < nb;
     int b = b0;
-    float acc = 0.f;
+    float acc[NC] = {};
     if (any) issue(tile, b0);
-    q45_prep(xc, nb, xlds);  // the first loads are in flight meanwhile
+    q45_prep<NC>(a, c0, nb, xlds);  // the first loads are in flight meanwhile
     __syncthreads();
     for (;;) {
         if (!any) {  // SH only
-            finish(0.f, tile);
+            finish(acc, tile);
             tile += g8;
             if (tile >= tiles) break;
             continue;
@@ -1059,12 +1143,15 @@ __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
         scale_min_k4(2 * g, P.y, P.z, P.w, s0, m0);
         scale_min_k4(2 * g + 1, P.y, P.z, P.w, s1, m1);
         const uint8_t *xb = xlds + b * kQ45Unit;
-        const float4 xs = *reinterpret_cast<const float4 *>(xb + 4 * kQ3Run + 16 * g);
-        const float4 xx = *reinterpret_cast<const float4 *>(xb + 4 * kQ3Run + 64 + 16 * g);
-        float ad = 0.f, am = 0.f;
+        f32x4 xs[NC], xx[NC];
+        float ad[NC] = {}, am[NC] = {};
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {  // column i: nb units further each
+            xs[i] = *reinterpret_cast<const f32x4 *>(xb + i * nb * kQ45Unit + 4 * kQ3Run + 16 * g);
+            xx[i] = *reinterpret_cast<const f32x4 *>(xb + i * nb * kQ45Unit + 4 * kQ3Run + 64 + 16 * g);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + kQ3Run * j + aoff);
             const u32x4 &q = (j & 1) ? q1 : q0;
             q3v4i Bc;
 #pragma unroll
@@ -1076,17 +1163,19 @@ __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
                 }
                 Bc[d] = static_cast<int>(v);
             }
-            const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, Bc, q3v4i{0, 0, 0, 0}, 0, 0, 0);
-            const int U = (D[0] << 16) + (D[1] << 8) + D[2];
-            const float xsj = j == 0 ? xs.x : j == 1 ? xs.y : j == 2 ? xs.z : xs.w;
-            const float xxj = j == 0 ? xx.x : j == 1 ? xx.y : j == 2 ? xx.z : xx.w;
-            ad = __builtin_fmaf(static_cast<float>(j < 2 ? s0 : s1), xsj * static_cast<float>(U), ad);
-            am = __builtin_fmaf(static_cast<float>(j < 2 ? m0 : m1), xxj, am);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + i * nb * kQ45Unit + kQ3Run * j + aoff);
+                const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, Bc, q3v4i{0, 0, 0, 0}, 0, 0, 0);
+                const int U = (D[0] << 16) + (D[1] << 8) + D[2];
+                ad[i] = __builtin_fmaf(static_cast<float>(j < 2 ? s0 : s1), xs[i][j] * static_cast<float>(U), ad[i]);
+                am[i] = __builtin_fmaf(static_cast<float>(j < 2 ? m0 : m1), xx[i][j], am[i]);
+            }
         }
-        acc += f16f(P.x & 0xffffu) * ad - f16f(P.x >> 16) * am;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) acc[i] += f16f(P.x & 0xffffu) * ad[i] - f16f(P.x >> 16) * am[i];
         if (last) {
             finish(acc, tile);
-            acc = 0.f;
             b = b0;
             tile += g8;
         } else {
@@ -1111,13 +1200,13 @@ __global__ __launch_bounds__(kQ3Threads) void kq45_mfma_kernel(KqArgs a) {
 // plane sums can pass 2^31 combined, so U is combined in fp32.
 constexpr int kQ8Seg = 272;  // segment bytes of a row (8 blocks)
 
+template <int NC>
 __global__ __launch_bounds__(kQ3Threads) void kq8_mfma_kernel(KqArgs a) {
 #pragma clang fp contract(off)
     constexpr int NU = kQ8Seg / 16, kUnits = 16 * NU, kIns = (kUnits + 63) / 64;
     extern __shared__ __attribute__((aligned(16))) uint8_t xlds[];
     const int nb = a.in_len / 256;  // steps: 256-element chunks
-    const int col = blockIdx.y;
-    const float *xc = a.x + static_cast<long long>(col) * a.in_len;
+    const int c0 = blockIdx.y * NC;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
     const int aoff = (c >> 2) == g && (c & 3) < 3 ? 48 * g + 16 * (c & 3) : 192;
@@ -1126,9 +1215,9 @@ __global__ __launch_bounds__(kQ3Threads) void kq8_mfma_kernel(KqArgs a) {
     if (tile >= tiles) return;  // the whole workgroup (blockIdx.x is uniform)
     const uint32_t rb32 = static_cast<uint32_t>(a.row_bytes);
     const int g8 = gridDim.x;
-    uint8_t *wl = xlds + nb * kQ45Unit + wave * (16 * kQ8Seg);
-    // the wavefronts' row sums [tile parity][wavefront][row], after the staging areas
-    float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + nb * kQ45Unit + 4 * 16 * kQ8Seg);
+    uint8_t *wl = xlds + NC * nb * kQ45Unit + wave * (16 * kQ8Seg);
+    // the wavefronts' row sums [tile parity, column][wavefront][row], after the staging areas
+    float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + NC * nb * kQ45Unit + 4 * 16 * kQ8Seg);
     int urow[kIns], uoff[kIns];
 #pragma unroll
     for (int i = 0; i < kIns; ++i) {
@@ -1151,18 +1240,9 @@ __global__ __launch_bounds__(kQ3Threads) void kq8_mfma_kernel(KqArgs a) {
         for (int i = 0; i < kIns; ++i)
             if (64 * i + lane < kUnits) *reinterpret_cast<u32x4 *>(wl + kQ8Seg * urow[i] + uoff[i]) = st[i];
     };
-    auto finish = [&](float acc, int t) {  // every wavefront, once a tile
-        auto q1 = __builtin_amdgcn_permlane32_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q1[0]) + fbits(q1[1]);
-        auto q2 = __builtin_amdgcn_permlane16_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q2[0]) + fbits(q2[1]);
-        const int par = (t / g8) & 1;
-        if (g == 0) red[par][wave][c] = acc;
-        __syncthreads();
-        const int row = t * 16 + c;
-        if (wave == 0 && g == 0 && row < a.out_len)
-            a.y[static_cast<long long>(col) * a.out_len + row] =
-                ((red[par][0][c] + red[par][1][c]) + red[par][2][c]) + red[par][3][c];
+    auto finish = [&](float (&acc)[NC], int t) {
+        finish_sh<NC>(a, red, (t / g8) & 1, acc, t, c0, wave, lane);
+        zero(acc);
     };
     // the lane's blocks 2g (codes from segment byte 68 g + 2) and 2g + 1
     // (d at 68 g + 34, codes from 68 g + 36)
@@ -1170,13 +1250,13 @@ __global__ __launch_bounds__(kQ3Threads) void kq8_mfma_kernel(KqArgs a) {
     const int s0 = wave;
     const bool any = s0 < nb;  // wavefronts without steps only meet the others at the tile's end
     int s = s0;
-    float acc = 0.f;
+    float acc[NC] = {};
     if (any) issue(tile, s0);
-    q45_prep(xc, nb, xlds);  // the first loads are in flight meanwhile
+    q45_prep<NC>(a, c0, nb, xlds);  // the first loads are in flight meanwhile
     __syncthreads();
     for (;;) {
         if (!any) {
-            finish(0.f, tile);
+            finish(acc, tile);
             tile += g8;
             if (tile >= tiles) break;
             continue;
@@ -1196,23 +1276,27 @@ __global__ __launch_bounds__(kQ3Threads) void kq8_mfma_kernel(KqArgs a) {
         }
         const float de = f16f(w[0] & 0xffffu), dodd = f16f(w[8] >> 16);
         const uint8_t *xb = xlds + s * kQ45Unit;
-        const float4 xs = *reinterpret_cast<const float4 *>(xb + 4 * kQ3Run + 16 * g);
-        float be = 0.f, bo = 0.f;
+        f32x4 xs[NC];
+        float be[NC] = {}, bo[NC] = {};
+#pragma unroll
+        for (int i = 0; i < NC; ++i) xs[i] = *reinterpret_cast<const f32x4 *>(xb + i * nb * kQ45Unit + 4 * kQ3Run + 16 * g);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + kQ3Run * j + aoff);
             const u32x4 &q = j < 2 ? ce[j & 1] : co[j & 1];
             const q3v4i Bc{static_cast<int>(q.x), static_cast<int>(q.y), static_cast<int>(q.z), static_cast<int>(q.w)};
-            const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, Bc, q3v4i{0, 0, 0, 0}, 0, 0, 0);
-            const float U = __builtin_fmaf(static_cast<float>(D[0]), 65536.f, static_cast<float>((D[1] << 8) + D[2]));
-            const float xsj = j == 0 ? xs.x : j == 1 ? xs.y : j == 2 ? xs.z : xs.w;
-            if (j < 2) be = __builtin_fmaf(xsj, U, be);
-            else bo = __builtin_fmaf(xsj, U, bo);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + i * nb * kQ45Unit + kQ3Run * j + aoff);
+                const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, Bc, q3v4i{0, 0, 0, 0}, 0, 0, 0);
+                const float U = __builtin_fmaf(static_cast<float>(D[0]), 65536.f, static_cast<float>((D[1] << 8) + D[2]));
+                if (j < 2) be[i] = __builtin_fmaf(xs[i][j], U, be[i]);
+                else bo[i] = __builtin_fmaf(xs[i][j], U, bo[i]);
+            }
         }
-        acc += de * be + dodd * bo;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) acc[i] += de * be[i] + dodd * bo[i];
         if (last) {
             finish(acc, tile);
-            acc = 0.f;
             s = s0;
             tile += g8;
         } else {
@@ -1244,8 +1328,9 @@ __global__ __launch_bounds__(kQ3Threads) void kq8_mfma_kernel(KqArgs a) {
 // the order the odd blocks' x planes are stored in).
 constexpr int kQ6Pitch = 432;  // LDS bytes of a staged row (420 used)
 
-template <int PAR>  // 0: the step's even block, 1: its odd block
-__device__ __forceinline__ float q6_block(const uint8_t *rl, const uint8_t *xb, int aoff, int n, int h, int g) {
+template <int PAR, int NC>  // PAR 0: the step's even block, 1: its odd block; xstep: LDS bytes between columns
+__device__ __forceinline__ void q6_block(const uint8_t *rl, const uint8_t *xb, int xstep, int aoff, int n, int h, int g,
+                                         float (&out)[NC]) {
 #pragma clang fp contract(off)
     constexpr int B0 = PAR ? 210 : 0;  // the block's first byte in the LDS row
     u32x4 l0v, l1v, qh;
@@ -1277,11 +1362,12 @@ __device__ __forceinline__ float q6_block(const uint8_t *rl, const uint8_t *xb, 
         sc.y = __builtin_amdgcn_alignbyte(s2, s1, 2);
         d = f16f(*reinterpret_cast<const uint16_t *>(rl + B0 + 208));
     }
-    const float4 xs = *reinterpret_cast<const float4 *>(xb + 4 * kQ3Run + 16 * g);
-    float blk = 0.f;
+    f32x4 xs[NC];
+    float blk[NC] = {};
+#pragma unroll
+    for (int i = 0; i < NC; ++i) xs[i] = *reinterpret_cast<const f32x4 *>(xb + i * xstep + 4 * kQ3Run + 16 * g);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + kQ3Run * j + aoff);
         const u32x4 &ql = (j & 1) ? l1v : l0v;
         q3v4i Bc;
 #pragma unroll
@@ -1290,24 +1376,27 @@ __device__ __forceinline__ float q6_block(const uint8_t *rl, const uint8_t *xb, 
             const uint32_t hi = __builtin_amdgcn_alignbit(qh[dw], qh[dw], static_cast<uint32_t>(2 * j - 6) & 31u) & 0xc0c0c0c0u;
             Bc[dw] = static_cast<int>((lo | hi) ^ 0x80808080u);
         }
-        const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, Bc, q3v4i{0, 0, 0, 0}, 0, 0, 0);
-        // 4 (65536 S0 + 256 S1 + S2): each plane sum a multiple of 4
-        const float U = __builtin_fmaf(static_cast<float>(D[0]), 16384.f, static_cast<float>((D[1] << 6) + (D[2] >> 2)));
         const int scj = __builtin_amdgcn_sbfe(static_cast<int>(j < 2 ? sc.x : sc.y), 8 * h + 16 * (j & 1), 8);
-        const float xsj = j == 0 ? xs.x : j == 1 ? xs.y : j == 2 ? xs.z : xs.w;
-        blk = __builtin_fmaf(static_cast<float>(scj), xsj * U, blk);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const q3v4i A = *reinterpret_cast<const q3v4i *>(xb + i * xstep + kQ3Run * j + aoff);
+            const q3v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, Bc, q3v4i{0, 0, 0, 0}, 0, 0, 0);
+            // 4 (65536 S0 + 256 S1 + S2): each plane sum a multiple of 4
+            const float U = __builtin_fmaf(static_cast<float>(D[0]), 16384.f, static_cast<float>((D[1] << 6) + (D[2] >> 2)));
+            blk[i] = __builtin_fmaf(static_cast<float>(scj), xs[i][j] * U, blk[i]);
+        }
     }
-    return d * blk;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) out[i] = d * blk[i];
 }
 
-template <int KIND, bool SH>  // SH: the shared 16-row tiles of kq45_mfma_kernel
+template <bool SH, int NC>  // SH: the shared 16-row tiles of kq45_mfma_kernel
 __global__ __launch_bounds__(kQ3Threads) void kq6_mfma_kernel(KqArgs a) {
     constexpr int kUnits = 16 * 26, kIns = (kUnits + 63) / 64;
     constexpr int RT = SH ? 16 : kQ3Rows;  // rows a tile
     extern __shared__ __attribute__((aligned(16))) uint8_t xlds[];
     const int nb = a.in_len / 256, steps = nb / 2;
-    const int col = blockIdx.y;
-    const float *xc = a.x + static_cast<long long>(col) * a.in_len;
+    const int c0 = blockIdx.y * NC;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4, n = g >> 1, h = g & 1;
     const int aoff = (c >> 2) == g && (c & 3) < 3 ? 48 * g + 16 * (c & 3) : 192;
@@ -1317,8 +1406,8 @@ __global__ __launch_bounds__(kQ3Threads) void kq6_mfma_kernel(KqArgs a) {
     if (tile >= tiles) return;  // the whole workgroup (blockIdx.x is uniform)
     const uint32_t rb32 = static_cast<uint32_t>(a.row_bytes);
     const int g8 = gridDim.x;
-    uint8_t *wl = xlds + nb * kQ3Unit + wave * (16 * kQ6Pitch);
-    float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + nb * kQ3Unit + 4 * 16 * kQ6Pitch);
+    uint8_t *wl = xlds + NC * nb * kQ3Unit + wave * (16 * kQ6Pitch);
+    float(*red)[4][16] = reinterpret_cast<float(*)[4][16]>(xlds + NC * nb * kQ3Unit + 4 * 16 * kQ6Pitch);
     int urow[kIns], uoff[kIns];
 #pragma unroll
     for (int i = 0; i < kIns; ++i) {
@@ -1345,23 +1434,10 @@ __global__ __launch_bounds__(kQ3Threads) void kq6_mfma_kernel(KqArgs a) {
             if (64 * i + lane < kUnits) *reinterpret_cast<u32x4 *>(wl + kQ6Pitch * urow[i] + uoff[i]) = st[i];
         if (lane < 16) *reinterpret_cast<uint32_t *>(wl + kQ6Pitch * lane + 416) = tail;
     };
-    auto finish = [&](float acc, int t) {
-        auto q1 = __builtin_amdgcn_permlane32_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q1[0]) + fbits(q1[1]);
-        auto q2 = __builtin_amdgcn_permlane16_swap(ubits(acc), ubits(acc), false, false);
-        acc = fbits(q2[0]) + fbits(q2[1]);
-        if constexpr (SH) {  // every wavefront, once a tile
-            const int par = (t / g8) & 1;
-            if (g == 0) red[par][wave][c] = acc;
-            __syncthreads();
-            const int row = t * RT + c;
-            if (wave == 0 && g == 0 && row < a.out_len)
-                a.y[static_cast<long long>(col) * a.out_len + row] =
-                    ((red[par][0][c] + red[par][1][c]) + red[par][2][c]) + red[par][3][c];
-        } else {
-            const int row = t * RT + rw + c;
-            if (g == 0 && row < a.out_len) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
-        }
+    auto finish = [&](float (&acc)[NC], int t) {
+        if constexpr (SH) finish_sh<NC>(a, red, (t / g8) & 1, acc, t, c0, wave, lane);
+        else finish_own<NC>(a, acc, t * RT + rw + c, c0, lane);
+        zero(acc);
     };
     const uint8_t *rl = wl + kQ6Pitch * c;
     // the wavefront's steps of a tile: s0, s0 + ss, .. (SH: wavefronts with
@@ -1369,13 +1445,13 @@ __global__ __launch_bounds__(kQ3Threads) void kq6_mfma_kernel(KqArgs a) {
     const int s0 = SH ? wave : 0, ss = SH ? 4 : 1;
     const bool any = !SH || s0 < steps;
     int s = s0;
-    float acc = 0.f;
+    float acc[NC] = {};
     if (any) issue(tile, s0);
-    q3_prep(xc, nb, xlds, 14);  // the first loads are in flight meanwhile
+    q3_prep<NC>(a, c0, nb, xlds, 14);  // the first loads are in flight meanwhile
     __syncthreads();
     for (;;) {
         if (!any) {  // SH only
-            finish(0.f, tile);
+            finish(acc, tile);
             tile += g8;
             if (tile >= tiles) break;
             continue;
@@ -1384,11 +1460,13 @@ __global__ __launch_bounds__(kQ3Threads) void kq6_mfma_kernel(KqArgs a) {
         const bool last = s + ss >= steps;
         issue(last ? tile + g8 : tile, last ? s0 : s + ss);
         __builtin_amdgcn_sched_barrier(0);
-        acc += q6_block<0>(rl, xlds + 2 * s * kQ3Unit, aoff, n, h, g);
-        acc += q6_block<1>(rl, xlds + (2 * s + 1) * kQ3Unit, aoff, n, h, g);
+        float v[NC];
+        q6_block<0, NC>(rl, xlds + 2 * s * kQ3Unit, nb * kQ3Unit, aoff, n, h, g, v);
+        add(acc, v);
+        q6_block<1, NC>(rl, xlds + (2 * s + 1) * kQ3Unit, nb * kQ3Unit, aoff, n, h, g, v);
+        add(acc, v);
         if (last) {
             finish(acc, tile);
-            acc = 0.f;
             s = s0;
             tile += g8;
         } else {
@@ -1415,6 +1493,12 @@ int cu_count() {
     });
     return n;
 }
+
+// Threads a CU of the task kernel's grid.  Each workgroup converts x once and
+// walks its tiles; what does not fit on the chip at once converts it for
+// nothing (4096x14336 Q6_K, one column: 2048 threads a CU 16.3, 1024 13.2, 512
+// 12.8 us; six columns, three at a time, 77 / 56 / 46 us).
+constexpr int kTaskThreads = 512;
 
 // Launch shape for rows of tpr tasks: slots side by side in a workgroup of
 // nt threads (up to 256 threads, the most rows side by side with the fewest
@@ -1454,7 +1538,8 @@ KqPlan kq_plan(int tpr) {
 // faster (Q3_K 4096x14336 20.3 against 26.4 us; 1024x5120 4.2-5.2 against
 // 12.0-13.2 us).  Other Q4_K measurements: 8192x8192 23.4 -> 11.8,
 // 4096x14336 38.1 -> 15.5, 6912x2560 9.1 -> 6.0 us with SH.
-constexpr int kShRed = 2 * 4 * 16 * 4;  // LDS bytes of SH's row sums
+constexpr int kShRed = 2 * 4 * 16 * 4;  // LDS bytes of SH's row sums of a column
+constexpr size_t kLdsMax = 160 * 1024;
 int kq_tiling(int out_len, size_t lds, int steps, bool any_sh) {
     if (lds > 65536) return -1;
     const int t64 = (out_len + kQ3Rows - 1) / kQ3Rows, cus = cu_count();
@@ -1465,50 +1550,88 @@ int kq_tiling(int out_len, size_t lds, int steps, bool any_sh) {
     return 0;
 }
 
+// Columns a workgroup takes at once (1..4) for k of them: the least work, a
+// pass over the codes (load and decode) costing about one column's products
+// and conversion of x, among the counts that LDS holds (fit) and that leave
+// enough workgroups: tiles * column groups >= wgs.  Columns one by one then
+// overlap better (Q6_K 300x2560, 4 columns: 4.3 us, as one group 9.2).
+// Measured, one by one -> grouped: Q6_K 8192x8192 2 / 4 columns 24.8 / 45.3 ->
+// 16.9 / 25.2 us, 20000x3072 9 columns 77 -> 50; Q4_K there 13.0 / 22.6 ->
+// 13.5 / 22.1 and 45 -> 31 us.
+int kq_columns(int k, int fit, long long tiles, long long wgs) {
+    int best = 1, cost = 2 * k;
+    for (int nc = 2; nc <= std::min(4, fit); ++nc) {
+        const int groups = (k + nc - 1) / nc, c = groups * (1 + nc);
+        if (c < cost && tiles * groups >= wgs) best = nc, cost = c;
+    }
+    return best;
+}
+
+// Launches pick(columns), the kernel for a column count, where x's planes take
+// `planes` bytes of LDS a column and the staging areas `rest`; cap: workgroups
+// per CU at most.  Planes of over 40 KiB a column stay one by one: a group of
+// them leaves one workgroup of four wavefronts a CU (Q4_K 4096x14336, 6
+// columns: 37 us one by one, 50 in pairs).
+template <class Pick>
+int launch_mfma(const char *what, Pick pick, const KqArgs &a, int tiles, int cap, size_t planes, size_t rest, bool sh,
+                hipStream_t s) {
+    const size_t red = sh ? kShRed : 0;
+    const int fit = planes > 40 * 1024 ? 1 : static_cast<int>((kLdsMax - rest) / (planes + red));
+    const int nc = kq_columns(a.k, fit, tiles, 2LL * cu_count());
+    const size_t lds = nc * (planes + red) + rest;
+    void (*fn)(KqArgs) = nc == 1 ? pick(std::integral_constant<int, 1>{})
+                         : nc == 2 ? pick(std::integral_constant<int, 2>{})
+                         : nc == 3 ? pick(std::integral_constant<int, 3>{})
+                                   : pick(std::integral_constant<int, 4>{});
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        if (e != hipSuccess) return fail(OURO_ERR_HIP, "%s: %zu B of LDS refused: %s", what, lds, hipGetErrorString(e));
+    }
+    if (nc > 1) cap = std::min(cap, static_cast<int>(kLdsMax / lds));  // no more than fit: each converts x anew
+    const dim3 grid(std::min(tiles, cu_count() * cap), (a.k + nc - 1) / nc);
+    hipLaunchKernelGGL(fn, grid, dim3(kQ3Threads), lds, s, a);
+    return check_launch(what);
+}
+
 template <int KIND>
-int launch_kind(KqArgs a, int k, bool al16, hipStream_t s) {
+int launch_kind(KqArgs a, bool al16, hipStream_t s) {
     const bool ph = a.row_bytes % 4 == 0;
+    const int t16 = (a.out_len + 15) / 16, t64 = (a.out_len + kQ3Rows - 1) / kQ3Rows;
     using F = Fmt<KIND>;
     if constexpr (KIND == OURO_KIND_Q8_0) {
         // a 16-byte-aligned payload with rows of a multiple of 8 blocks
         const int nb = a.in_len / 256;
-        const size_t lds = static_cast<size_t>(nb) * kQ45Unit + kQ3Waves * 16 * kQ8Seg;
-        if (al16 && a.in_len % 256 == 0 && kq_tiling(a.out_len, lds, nb, true) == 1) {
-            const dim3 grid(std::min((a.out_len + 15) / 16, cu_count() * 4), k);
-            hipLaunchKernelGGL(kq8_mfma_kernel, grid, dim3(kQ3Threads), lds + kShRed, s, a);
-            return check_launch("kq8_mfma_kernel");
-        }
+        const size_t planes = static_cast<size_t>(nb) * kQ45Unit, rest = kQ3Waves * 16 * kQ8Seg;
+        if (al16 && a.in_len % 256 == 0 && kq_tiling(a.out_len, planes + rest, nb, true) == 1)
+            return launch_mfma("kq8_mfma_kernel", [](auto n) { return kq8_mfma_kernel<decltype(n)::value>; }, a, t16, 4,
+                               planes, rest, true, s);
     }
     if constexpr (KIND == OURO_KIND_Q6K) {
         // dword-aligned payload and rows (nb even): steps of an even and an odd block
         const int nb = a.in_len / 256;
-        const size_t lds = static_cast<size_t>(nb) * kQ3Unit + kQ3Waves * 16 * kQ6Pitch;
-        const int til = kq_tiling(a.out_len, lds, nb / 2, true);
+        const size_t planes = static_cast<size_t>(nb) * kQ3Unit, rest = kQ3Waves * 16 * kQ6Pitch;
+        const int til = kq_tiling(a.out_len, planes + rest, nb / 2, true);
         if (reinterpret_cast<uintptr_t>(a.w) % 4 == 0 && ph && til >= 0) {
-            if (til == 1) {
-                const dim3 grid(std::min((a.out_len + 15) / 16, cu_count() * 3), k);
-                hipLaunchKernelGGL((kq6_mfma_kernel<KIND, true>), grid, dim3(kQ3Threads), lds + kShRed, s, a);
-            } else {
-                const dim3 grid(std::min((a.out_len + kQ3Rows - 1) / kQ3Rows, cu_count() * 3), k);
-                hipLaunchKernelGGL((kq6_mfma_kernel<KIND, false>), grid, dim3(kQ3Threads), lds, s, a);
-            }
-            return check_launch("kq6_mfma_kernel");
+            if (til == 1)
+                return launch_mfma("kq6_mfma_kernel", [](auto n) { return kq6_mfma_kernel<true, decltype(n)::value>; }, a,
+                                   t16, 3, planes, rest, true, s);
+            return launch_mfma("kq6_mfma_kernel", [](auto n) { return kq6_mfma_kernel<false, decltype(n)::value>; }, a, t64,
+                               3, planes, rest, false, s);
         }
     }
     if constexpr (KIND == OURO_KIND_Q4K || KIND == OURO_KIND_Q5K) {
         // the matrix-core kernel on a 16-byte-aligned payload (every block and row then is)
         const int nb = a.in_len / 256;
-        const size_t lds = static_cast<size_t>(nb) * kQ45Unit + kQ3Waves * 16 * F::BB;
-        const int til = kq_tiling(a.out_len, lds, nb, true);
+        const size_t planes = static_cast<size_t>(nb) * kQ45Unit, rest = kQ3Waves * 16 * F::BB;
+        const int til = kq_tiling(a.out_len, planes + rest, nb, true);
         if (al16 && til >= 0) {
-            if (til == 1) {
-                const dim3 grid(std::min((a.out_len + 15) / 16, cu_count() * 4), k);
-                hipLaunchKernelGGL((kq45_mfma_kernel<KIND, true>), grid, dim3(kQ3Threads), lds + kShRed, s, a);
-            } else {
-                const dim3 grid(std::min((a.out_len + kQ3Rows - 1) / kQ3Rows, cu_count() * 4), k);
-                hipLaunchKernelGGL((kq45_mfma_kernel<KIND, false>), grid, dim3(kQ3Threads), lds, s, a);
-            }
-            return check_launch("kq45_mfma_kernel");
+            if (til == 1)
+                return launch_mfma("kq45_mfma_kernel",
+                                   [](auto n) { return kq45_mfma_kernel<KIND, true, decltype(n)::value>; }, a, t16, 4,
+                                   planes, rest, true, s);
+            return launch_mfma("kq45_mfma_kernel", [](auto n) { return kq45_mfma_kernel<KIND, false, decltype(n)::value>; },
+                               a, t64, 4, planes, rest, false, s);
         }
     }
     if constexpr (KIND == OURO_KIND_Q3K) {
@@ -1516,48 +1639,52 @@ int launch_kind(KqArgs a, int k, bool al16, hipStream_t s) {
         if (nb <= kQ3MaxBlocks) {
             // dword-aligned payload and rows (so nb is even): the staged loads
             const bool al = reinterpret_cast<uintptr_t>(a.w) % 4 == 0 && ph;
-            const int tiles = (a.out_len + kQ3Rows - 1) / kQ3Rows;
-            const dim3 grid(std::min(tiles, cu_count() * 4), k);
-            const size_t lds = static_cast<size_t>(nb) * kQ3Unit;
-            const size_t lds_st = lds + kQ3Waves * kQ3Stage;
-            const int til = al ? kq_tiling(a.out_len, lds_st, nb / 2, false) : -1;
-            if (til == 1) {
-                const dim3 gs(std::min((a.out_len + 15) / 16, cu_count() * 4), k);
-                hipLaunchKernelGGL(kq3_mfma_kernel<Q3K_STS>, gs, dim3(kQ3Threads), lds_st + kShRed, s, a);
-                return check_launch("kq3_mfma_kernel");
-            }
-            if (til == 0) {
-                hipLaunchKernelGGL(kq3_mfma_kernel<Q3K_ST>, grid, dim3(kQ3Threads), lds_st, s, a);
-                return check_launch("kq3_mfma_kernel");
-            }
-            if (!al && kq_tiling(a.out_len, lds, nb, false) == 0) {  // unstaged: each lane loads its own pieces
-                hipLaunchKernelGGL(kq3_mfma_kernel<Q3K_ANY>, grid, dim3(kQ3Threads), lds, s, a);
-                return check_launch("kq3_mfma_kernel");
-            }
+            const size_t planes = static_cast<size_t>(nb) * kQ3Unit, rest = kQ3Waves * kQ3Stage;
+            const int til = al ? kq_tiling(a.out_len, planes + rest, nb / 2, false) : -1;
+            if (til == 1)
+                return launch_mfma("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_STS, decltype(n)::value>; }, a,
+                                   t16, 4, planes, rest, true, s);
+            if (til == 0)
+                return launch_mfma("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_ST, decltype(n)::value>; }, a,
+                                   t64, 4, planes, rest, false, s);
+            if (!al && kq_tiling(a.out_len, planes, nb, false) == 0)  // unstaged: each lane loads its own pieces
+                return launch_mfma("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_ANY, decltype(n)::value>; }, a,
+                                   t64, 4, planes, 0, false, s);
         }
     }
     a.tpr = a.in_len / F::EPB * F::TPB;
     const KqPlan pl = kq_plan(a.tpr);
     if (!pl.slots) {
-        dim3 grid((a.out_len + 3) / 4, k);
+        dim3 grid((a.out_len + 3) / 4, a.k);
         hipLaunchKernelGGL(kq_row_kernel<KIND>, grid, dim3(256), 0, s, a);
         return check_launch("kq_row_kernel");
     }
     a.slots = pl.slots;
     const int nt = pl.nt;
-    auto go = [&](auto rows_c, auto maxt_c) {
-        constexpr int R = decltype(rows_c)::value, MAXT = decltype(maxt_c)::value;
+    auto go = [&](auto rows_c, auto maxt_c, auto cols_c) {
+        constexpr int R = decltype(rows_c)::value, MAXT = decltype(maxt_c)::value, NC = decltype(cols_c)::value;
         a.tiles = (a.out_len + a.slots * R - 1) / (a.slots * R);
-        const int grid_x = std::min(a.tiles, cu_count() * std::max(1, 2048 / nt));
-        const size_t lds = (a.slots == 1 ? static_cast<size_t>(kBatch1) * R * (nt / 64)
-                                         : static_cast<size_t>(kBatch) * R * nt) * sizeof(float);
-        dim3 grid(grid_x, k);
-        if (al16) hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, true, false, MAXT>), grid, dim3(nt), lds, s, a);
-        else if (ph) hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, true, MAXT>), grid, dim3(nt), lds, s, a);
-        else hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, false, MAXT>), grid, dim3(nt), lds, s, a);
+        const int grid_x = std::min(a.tiles, cu_count() * std::max(1, kTaskThreads / nt));
+        const size_t lds = (a.slots == 1 ? static_cast<size_t>(kBatch1 / NC * NC) * R * (nt / 64)
+                                         : static_cast<size_t>(kBatch / NC * NC) * R * nt) * sizeof(float);
+        dim3 grid(grid_x, (a.k + NC - 1) / NC);
+        if (al16) hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, true, false, MAXT, NC>), grid, dim3(nt), lds, s, a);
+        else if (ph) hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, true, MAXT, NC>), grid, dim3(nt), lds, s, a);
+        else hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, false, MAXT, NC>), grid, dim3(nt), lds, s, a);
     };
-    if (nt <= 512) go(std::integral_constant<int, kRows<KIND>>{}, std::integral_constant<int, 512>{});
-    else go(std::integral_constant<int, 1>{}, std::integral_constant<int, kMaxThreads>{});
+    constexpr std::integral_constant<int, kRows<KIND>> rows{};
+    constexpr std::integral_constant<int, 512> t512{};
+    if (nt > 512) {  // 1024 threads leave no registers for a second column's x
+        go(std::integral_constant<int, 1>{}, std::integral_constant<int, kMaxThreads>{}, std::integral_constant<int, 1>{});
+    } else {
+        const int t1 = (a.out_len + a.slots * 2 - 1) / (a.slots * 2);
+        switch (kq_columns(a.k, 4, t1, cu_count() * std::max(1, 1024 / nt) / 2)) {
+        case 1: go(rows, t512, std::integral_constant<int, 1>{}); break;
+        case 2: go(std::integral_constant<int, 2>{}, t512, std::integral_constant<int, 2>{}); break;
+        case 3: go(std::integral_constant<int, 2>{}, t512, std::integral_constant<int, 3>{}); break;
+        default: go(std::integral_constant<int, 2>{}, t512, std::integral_constant<int, 4>{}); break;
+        }
+    }
     return check_launch("kq_gemv_kernel");
 }
 
@@ -1596,13 +1723,13 @@ int kq_matmul(const void *payload, int kind, size_t out_len, size_t in_len, cons
     // the 144- and 176-byte blocks keep 16-byte alignment when the payload has it
     const bool al16 = reinterpret_cast<uintptr_t>(payload) % 16 == 0;
     const hipStream_t s = as_stream(stream);
-    const int kk = static_cast<int>(k);
+    a.k = static_cast<int>(k);
     switch (kind) {
-    case OURO_KIND_Q8_0: return launch_kind<OURO_KIND_Q8_0>(a, kk, al16, s);
-    case OURO_KIND_Q3K: return launch_kind<OURO_KIND_Q3K>(a, kk, false, s);
-    case OURO_KIND_Q4K: return launch_kind<OURO_KIND_Q4K>(a, kk, al16, s);
-    case OURO_KIND_Q5K: return launch_kind<OURO_KIND_Q5K>(a, kk, al16, s);
-    default: return launch_kind<OURO_KIND_Q6K>(a, kk, false, s);
+    case OURO_KIND_Q8_0: return launch_kind<OURO_KIND_Q8_0>(a, al16, s);
+    case OURO_KIND_Q3K: return launch_kind<OURO_KIND_Q3K>(a, false, s);
+    case OURO_KIND_Q4K: return launch_kind<OURO_KIND_Q4K>(a, al16, s);
+    case OURO_KIND_Q5K: return launch_kind<OURO_KIND_Q5K>(a, al16, s);
+    default: return launch_kind<OURO_KIND_Q6K>(a, false, s);
     }
 }
 

@@ -244,3 +244,33 @@ def test_kquant_shape_errors(gpu):
         call("ouro_matvec_q", p.ptr, int(QuantKind.Q8_0), 4, 48, x.ptr, y.ptr, None)
     with pytest.raises(OuroError):  # x misaligned
         call("ouro_matvec_q", p.ptr, int(QuantKind.Q6K), 4, 256, x.ptr + 2, y.ptr, None)
+
+
+@pytest.mark.parametrize("kind", KINDS, ids=lambda k: k.name)
+@pytest.mark.parametrize("out_len,in_len,offset", [(37, 768, 0), (97, 14336, 0), (300, 20480, 0), (2100, 768, 0),
+                                                   (2100, 1024, 2), (4100, 4096, 0), (8200, 8192, 0), (16399, 1536, 4),
+                                                   (16399, 10752, 0)])
+def test_kquant_column_groups(gpu, kind, out_len, in_len, offset):
+    """Columns are taken 1 to 4 at a time, by the task kernel and by each
+    tiling of the matrix-core kernels (planes of several columns past 64 KiB
+    of LDS among them); whatever the group, each column is the matvec of that
+    column bit for bit (which the tests above hold to the oracle), with a
+    ragged last group too."""
+    rng = np.random.default_rng(out_len + in_len + offset)
+    p = kq_payload(rng, kind, out_len, in_len)
+    buf = DeviceBuffer((p.size + 32,), np.uint8)
+    host = np.zeros(p.size + 32, np.uint8)
+    host[offset:offset + p.size] = p
+    buf.upload(host)
+    x = rng.standard_normal((11, in_len)).astype(np.float32)
+    xd, y = DeviceBuffer.from_host(x), DeviceBuffer((11, out_len), np.float32)
+    one = np.empty((11, out_len), np.float32)
+    for c in range(11):
+        call("ouro_matvec_q", buf.ptr + offset, int(kind), out_len, in_len, xd.ptr + 4 * c * in_len, y.ptr, None)
+        one[c] = y.download().reshape(11, out_len)[0]
+    for k in (2, 3, 4, 5, 6, 11):
+        y.upload(np.full((11, out_len), np.nan, np.float32))
+        call("ouro_matmul_q", buf.ptr + offset, int(kind), out_len, in_len, xd.ptr, k, y.ptr, None)
+        got = y.download().reshape(11, out_len)
+        assert np.array_equal(got[:k], one[:k]), k
+        assert np.isnan(got[k:]).all()
