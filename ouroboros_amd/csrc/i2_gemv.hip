@@ -122,13 +122,60 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const T *__restrict__ x,
     if (threadIdx.x == 0) act_scale[row] = s;
 }
 
+// The same for rows of whole 4-element groups, at most kQuantRegs a thread:
+// the row is read once, 4 elements a load, and stays in registers between the
+// maximum and the rounding; 4 bytes a store.  Bound by the bytes (1500x6912
+// f32: 52 MB, 24 us with the element loop above, 10.3 here).
+constexpr int kQuantRegs = 8;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+
+__device__ __forceinline__ f32x4 load_act4(const float *p) { return *reinterpret_cast<const f32x4_a4 *>(p); }
+__device__ __forceinline__ f32x4 load_act4(const uint16_t *p) {
+    const uint2 v = *reinterpret_cast<const uint2 *>(p);
+    return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                 __uint_as_float(v.y & 0xffff0000u)};
+}
+
+__device__ __forceinline__ uint32_t i8s_quant4(const f32x4 &v, float s) {
+    uint32_t q = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q |= (static_cast<uint32_t>(i8s_quant(v[i], s)) & 255u) << (8 * i);
+    return q;
+}
+
+template <typename T, int NV>
+__global__ __launch_bounds__(256) void act_quant4_kernel(const T *__restrict__ x, int n, int8_t *__restrict__ xq,
+                                                         float *__restrict__ act_scale) {
+    __shared__ float red[4];
+    const long long row = blockIdx.x;
+    const T *xr = x + row * n;
+    const int groups = n / 4;
+    f32x4 v[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = load_act4(xr + 4 * min(static_cast<int>(threadIdx.x) + 256 * j, groups - 1));
+    float amax = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(v[j][i]));
+    const float s = i8s_scale(block_max_256(amax, red));
+    uint32_t *qr = reinterpret_cast<uint32_t *>(xq + row * n);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int g = static_cast<int>(threadIdx.x) + 256 * j;
+        if (g < groups) qr[g] = i8s_quant4(v[j], s);
+    }
+    if (threadIdx.x == 0) act_scale[row] = s;
+}
+
 // ------------------------------------------------------------- GEMV --
 
 struct GemvArgs {
     const uint8_t *w;       // tiled codes of matrix 0
     long long w_stride;     // bytes between matrices
     const float *w_scale;   // per matrix, stride 1
-    const int8_t *xq;       // [ncols][in_len] of matrix 0
+    const int8_t *xq;       // [ncols][in_len] of matrix 0 (XF: f32 x [in_len])
     long long x_stride;     // elements between matrices
     const float *act_scale;    // [ncols] of matrix 0, per matrix stride ncols
     float *y;               // [ncols][out_len] of matrix 0
@@ -221,7 +268,11 @@ __device__ __forceinline__ int row_totals(int (&v)[R], int lane) {
 //              fields 1 and 3 at scale 4 (w & 0x0c.., (w >> 4) & 0x0c..),
 //              5 operations per word and two accumulators per row,
 //              recombined exactly as s1 + (s4 >> 2) (s4 is a multiple of 4).
-template <int G, int NC, int TPW, int DEPTH, int WPB, int SPLIT>
+// XF: xq is x itself in fp32 (one column): a wavefront's lanes hold a whole
+// row between them, so each wavefront takes the maximum and rounds its own
+// groups (as act_quant_kernel does, the same integers) and a decode step needs
+// no launch ahead of the product.
+template <int G, int NC, int TPW, int DEPTH, int WPB, int SPLIT, bool XF>
 __global__ __launch_bounds__(kWave *WPB) void i2_gemv_kernel(GemvArgs a) {
     constexpr int R = kTileRows;
     constexpr int U = unit_bytes(G);  // bytes per load
@@ -264,8 +315,31 @@ __global__ __launch_bounds__(kWave *WPB) void i2_gemv_kernel(GemvArgs a) {
     // load per chunk.
     uint32_t xw[NC][G];
     int sx[NC];
+    float xscale = 0.f;
+    if constexpr (XF) {
+        static_assert(NC == 1, "fp32 x: one column");
+        const float *xf = reinterpret_cast<const float *>(xq);
+        float amax = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
+        for (int g = 0; g < G; ++g) {
+            const f32x4 v = load_act4(xf + 4 * kgroup(G, lane, g));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(v[i]));
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, xor_shfl(amax, off));
+        xscale = i8s_scale(amax);
+        // a long row's second read comes from the cache, not from registers
+        if constexpr (G > 16) asm volatile("" ::: "memory");
+        sx[0] = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            xw[0][g] = i8s_quant4(load_act4(xf + 4 * kgroup(G, lane, g)), xscale);
+            sx[0] = __builtin_amdgcn_sdot4(static_cast<int>(xw[0][g]), 0x01010101, sx[0], false);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < (XF ? 0 : NC); ++c) {
         sx[c] = 0;
         const bool live = c0 + c < a.ncols;
         const uint32_t *xr = reinterpret_cast<const uint32_t *>(xq + static_cast<long long>(c0 + c) * a.in_len);
@@ -343,7 +417,7 @@ __global__ __launch_bounds__(kWave *WPB) void i2_gemv_kernel(GemvArgs a) {
             const int row = tile * R + lane / span;
             if (lane % span == span - 1 && row < a.out_len && c0 + c < a.ncols) {
                 const long long o = static_cast<long long>(c0 + c) * a.out_len + row;
-                const float v = i8s_out(total, act_scale[c0 + c], wscale);
+                const float v = i8s_out(total, XF ? xscale : act_scale[c0 + c], wscale);
                 y[o] = v;
                 if (a.acc) a.acc[o] = total;
             }
@@ -373,29 +447,29 @@ constexpr long long kGemvWaves = 2048;
 // only while 4 * G words of activations fit in 40 registers, NC = 2 while
 // 2 * G fit in 64.
 template <int G>
-GemvPick pick_g(int ncols, long long total_tiles) {
+GemvPick pick_g(int ncols, long long total_tiles, bool xf) {
     if constexpr (4 * G <= 40)
-        if (ncols >= 4) return {i2_gemv_kernel<G, 4, 1, 1, kGemvWpb, 1>, 4, 1, kGemvWpb};
+        if (ncols >= 4) return {i2_gemv_kernel<G, 4, 1, 1, kGemvWpb, 1, false>, 4, 1, kGemvWpb};
     if constexpr (2 * G <= 64)
-        if (ncols >= 2) return {i2_gemv_kernel<G, 2, 1, 1, kGemvWpb, 1>, 2, 1, kGemvWpb};
+        if (ncols >= 2) return {i2_gemv_kernel<G, 2, 1, 1, kGemvWpb, 1, false>, 2, 1, kGemvWpb};
     if constexpr (G <= 4)
-        if (total_tiles >= 2 * kGemvWaves) return {i2_gemv_kernel<G, 1, 2, 2, kGemvWpb, 2>, 1, 2, kGemvWpb};
-    return {i2_gemv_kernel<G, 1, 1, 1, kGemvWpb, 2>, 1, 1, kGemvWpb};
+        if (!xf && total_tiles >= 2 * kGemvWaves) return {i2_gemv_kernel<G, 1, 2, 2, kGemvWpb, 2, false>, 1, 2, kGemvWpb};
+    return {xf ? i2_gemv_kernel<G, 1, 1, 1, kGemvWpb, 2, true> : i2_gemv_kernel<G, 1, 1, 1, kGemvWpb, 2, false>, 1, 1, kGemvWpb};
 }
 
-GemvPick pick_gemv(int G, int ncols, long long total_tiles) {
+GemvPick pick_gemv(int G, int ncols, long long total_tiles, bool xf) {
     switch (G) {
-    case 1: return pick_g<1>(ncols, total_tiles);
-    case 2: return pick_g<2>(ncols, total_tiles);
-    case 4: return pick_g<4>(ncols, total_tiles);
-    case 8: return pick_g<8>(ncols, total_tiles);
-    case 10: return pick_g<10>(ncols, total_tiles);
-    case 12: return pick_g<12>(ncols, total_tiles);
-    case 16: return pick_g<16>(ncols, total_tiles);
-    case 20: return pick_g<20>(ncols, total_tiles);
-    case 24: return pick_g<24>(ncols, total_tiles);
-    case 27: return pick_g<27>(ncols, total_tiles);
-    case 32: return pick_g<32>(ncols, total_tiles);
+    case 1: return pick_g<1>(ncols, total_tiles, xf);
+    case 2: return pick_g<2>(ncols, total_tiles, xf);
+    case 4: return pick_g<4>(ncols, total_tiles, xf);
+    case 8: return pick_g<8>(ncols, total_tiles, xf);
+    case 10: return pick_g<10>(ncols, total_tiles, xf);
+    case 12: return pick_g<12>(ncols, total_tiles, xf);
+    case 16: return pick_g<16>(ncols, total_tiles, xf);
+    case 20: return pick_g<20>(ncols, total_tiles, xf);
+    case 24: return pick_g<24>(ncols, total_tiles, xf);
+    case 27: return pick_g<27>(ncols, total_tiles, xf);
+    case 32: return pick_g<32>(ncols, total_tiles, xf);
     default: return {nullptr, 0, 0, 0};
     }
 }
@@ -495,11 +569,11 @@ __global__ __launch_bounds__(kWave *kI2sWaves) void i2s_gemv_kernel(I2sArgs a) {
     }
 }
 
-int launch_gemv(const GemvArgs &base, int count, void *stream) {
+int launch_gemv(const GemvArgs &base, int count, void *stream, bool xf = false) {
     const int G = base.in_len / 256;
     const int tiles = base.tiles;
     const long long total_tiles = static_cast<long long>(tiles) * count;
-    const GemvPick p = pick_gemv(G, base.ncols, total_tiles);
+    const GemvPick p = pick_gemv(G, base.ncols, total_tiles, xf);
     if (!p.fn) return fail(OURO_ERR_SHAPE, "i2 gemv: in_len %d (G=%d) has no kernel instance", base.in_len, G);
     const int nc = p.nc;
     const int per_block = p.wpb * p.tpw;
@@ -546,18 +620,54 @@ int i2_gemm(const uint8_t *w_tiled, size_t out_len, size_t in_len, const float *
     return launch_gemv(a, 1, stream);
 }
 
+// y = W x for one fp32 column in one launch (the product quantises x itself).
+// Each wavefront does that for its 8 rows, some 32 operations per group of
+// four elements and lane: past kFusedGroups tiles * groups the separate launch is cheaper
+// (quantise + product -> fused: 6912x2560 7.7 -> 3.9, 2560x6912 12.8 -> 7.1,
+// 8192x8192 14.8 -> 9.1, 32768x2048, at the line, 8.0 -> 6.9 us).
+constexpr size_t kFusedGroups = 32768;
+bool i2_matvec_f32_pays(size_t out_len, size_t in_len) {
+    return (out_len + kTileRows - 1) / kTileRows * (in_len / 256) <= kFusedGroups;
+}
+int i2_matvec_f32(const uint8_t *w_tiled, size_t out_len, size_t in_len, const float *w_scale, const float *x, float *y,
+                  void *stream) {
+    const int st = check_i2_shape(out_len, in_len);
+    if (st) return st;
+    if (reinterpret_cast<uintptr_t>(w_tiled) % 16)
+        return fail(OURO_ERR_ALIGN, "ouro_gemm_i2: weights and xq need 16-byte alignment");
+    GemvArgs a{};
+    a.w = w_tiled;
+    a.w_scale = w_scale;
+    a.xq = reinterpret_cast<const int8_t *>(x);
+    a.y = y;
+    a.out_len = static_cast<int>(out_len);
+    a.in_len = static_cast<int>(in_len);
+    a.ncols = 1;
+    a.tiles = static_cast<int>((out_len + kTileRows - 1) / kTileRows);
+    return launch_gemv(a, 1, stream, true);
+}
+
+// act_quant4_kernel for rows of n elements, or the element loop.
+template <typename T>
+void launch_act_quant(const T *x, size_t rows, size_t n, int8_t *xq, float *act_scale, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(rows)), block(256);
+    const bool four = n % 4 == 0 && n <= 4 * 256 * kQuantRegs && reinterpret_cast<uintptr_t>(xq) % 4 == 0 &&
+                      reinterpret_cast<uintptr_t>(x) % (sizeof(T) == 2 ? 8 : 4) == 0;
+    const int m = static_cast<int>(n);
+    if (!four) hipLaunchKernelGGL(act_quant_kernel<T>, grid, block, 0, s, x, static_cast<long long>(n), xq, act_scale);
+    else if (n <= 2 * 1024) hipLaunchKernelGGL((act_quant4_kernel<T, 2>), grid, block, 0, s, x, m, xq, act_scale);
+    else if (n <= 4 * 1024) hipLaunchKernelGGL((act_quant4_kernel<T, 4>), grid, block, 0, s, x, m, xq, act_scale);
+    else hipLaunchKernelGGL((act_quant4_kernel<T, kQuantRegs>), grid, block, 0, s, x, m, xq, act_scale);
+}
+
 int act_quant(const void *x, int x_dtype, size_t rows, size_t n, int8_t *xq, float *act_scale,
               void *stream) {
     if (!x || !xq || !act_scale) return fail(OURO_ERR_INVALID_ARG, "ouro_act_quant_i8: NULL argument");
     if (!rows || !n) return fail(OURO_ERR_SHAPE, "ouro_act_quant_i8: empty shape");
     if (rows > 0x7fffffff) return fail(OURO_ERR_SHAPE, "ouro_act_quant_i8: too many rows");
-    dim3 grid(static_cast<unsigned>(rows)), block(256);
-    if (x_dtype == OURO_DT_F32)
-        hipLaunchKernelGGL(act_quant_kernel<float>, grid, block, 0, as_stream(stream),
-                           static_cast<const float *>(x), static_cast<long long>(n), xq, act_scale);
+    if (x_dtype == OURO_DT_F32) launch_act_quant(static_cast<const float *>(x), rows, n, xq, act_scale, as_stream(stream));
     else if (x_dtype == OURO_DT_BF16)
-        hipLaunchKernelGGL(act_quant_kernel<uint16_t>, grid, block, 0, as_stream(stream),
-                           static_cast<const uint16_t *>(x), static_cast<long long>(n), xq, act_scale);
+        launch_act_quant(static_cast<const uint16_t *>(x), rows, n, xq, act_scale, as_stream(stream));
     else
         return fail(OURO_ERR_INVALID_ARG, "ouro_act_quant_i8: bad dtype %d", x_dtype);
     return check_launch("act_quant_kernel");

@@ -23,6 +23,9 @@ int i2_gemm(const uint8_t *w_tiled, size_t out_len, size_t in_len, const float *
 int act_quant(const void *x, int x_dtype, size_t rows, size_t n, int8_t *xq, float *act_scale,
               void *stream);
 size_t i2_tiled_bytes(size_t out_len, size_t in_len);
+bool i2_matvec_f32_pays(size_t out_len, size_t in_len);
+int i2_matvec_f32(const uint8_t *w_tiled, size_t out_len, size_t in_len, const float *w_scale, const float *x, float *y,
+                  void *stream);
 int i2s_gemm(const uint8_t *i2s, size_t out_len, size_t in_len, const int8_t *xq, const float *act_scale,
              size_t ncols, float *y, int32_t *acc, void *stream);
 size_t tl1_lut_partial_floats(size_t out_len, size_t in_len);
@@ -262,6 +265,10 @@ int matmul_q(const void *payload, int kind, size_t out_len, size_t in_len, const
     case OURO_KIND_I2_S: {
         const size_t tb = i2_tiled_bytes(out_len, in_len);
         if (!tb) return fail(OURO_ERR_SHAPE, "matvec_q I2: in_len %zu not a multiple of 256", in_len);
+        if (kind == OURO_KIND_I2 && k == 1 && i2_matvec_f32_pays(out_len, in_len)) {  // one launch, no scratch
+            const uint8_t *w = static_cast<const uint8_t *>(payload);
+            return i2_matvec_f32(w, out_len, in_len, reinterpret_cast<const float *>(w + tb), x, y, stream);
+        }
         int8_t *xq = xq_scratch;
         float *ds = act_scale_scratch;
         if (!xq) {
