@@ -346,10 +346,11 @@ int run_layer(ouro_stack *s, int il, size_t rows, bool prefill, const int32_t *c
     return OURO_OK;
 }
 
-// Final norm of the chosen rows of the residual stream, lm_head, greedy token.
+// Final norm of the chosen rows of the residual stream (rows_idx NULL: rows
+// 0 .. n - 1 where they are), lm_head, greedy token.
 int head(ouro_stack *s, const int32_t *rows_idx, size_t n, int32_t *next, float *logits_out, void *stream) {
-    TRY(gather_rows(s->x, rows_idx, s->lp, n, s->E, stream));
-    TRY(rq(s, RQ_NORM, s->lp, nullptr, s->out_norm, nullptr, n, s->E, s->sign_e, stream));
+    if (rows_idx) TRY(gather_rows(s->x, rows_idx, s->lp, n, s->E, stream));
+    TRY(rq(s, RQ_NORM, rows_idx ? s->lp : s->x, nullptr, s->out_norm, nullptr, n, s->E, s->sign_e, stream));
     float *lg = logits_out ? logits_out : s->logits;
     TRY(lin(s->lm, n, s->xq, s->ds, lg, stream));
     return argmax_rows(lg, n, s->V, next, s->arg_keys, stream);
@@ -636,7 +637,7 @@ int ouro_stack_decode(ouro_stack_t s, const int32_t *tokens, int32_t *next_token
     s->max_len += 1;
     TRY(embed_rows(tokens, s->embd, s->x, B, s->V, s->E, stream));
     for (int il = 0; il < s->c.n_layer; ++il) TRY(run_layer(s, il, B, false, nullptr, B, 0, stream));
-    return head(s, s->dec_seq, B, next_tokens, logits_or_null, stream);
+    return head(s, nullptr, B, next_tokens, logits_or_null, stream);
 }
 
 }  // extern "C"
