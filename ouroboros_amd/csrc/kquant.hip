@@ -1497,7 +1497,7 @@ int cu_count() {
 // Threads a CU of the task kernel's grid.  Each workgroup converts x once and
 // walks its tiles; what does not fit on the chip at once converts it for
 // nothing (4096x14336 Q6_K, one column: 2048 threads a CU 16.3, 1024 13.2, 512
-// 12.8 us; six columns, three at a time, 77 / 56 / 46 us).
+// 12.8 us; six columns, three at a time, two rows a tile, 77 / 56 / 46 us).
 constexpr int kTaskThreads = 512;
 
 // Launch shape for rows of tpr tasks: slots side by side in a workgroup of
@@ -1674,15 +1674,26 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
     };
     constexpr std::integral_constant<int, kRows<KIND>> rows{};
     constexpr std::integral_constant<int, 512> t512{};
+    // Several columns: four rows a tile where that still gives every workgroup
+    // two tiles, else two (three columns of Q6_K, R = 2 / 4: 32768x1792 24.7 /
+    // 21.5, 4096x14336 24.1 / 21.5, 1500x7168 9.7 / 10.8 us).
+    auto cols = [&](auto cols_c) {
+        // four columns of Q3_K and Q5_K leave no registers for four rows
+        constexpr int R = decltype(cols_c)::value == 4 && (KIND == OURO_KIND_Q3K || KIND == OURO_KIND_Q5K) ? 2 : 4;
+        if ((a.out_len + a.slots * 4 - 1) / (a.slots * 4) >= 2 * cu_count() * std::max(1, kTaskThreads / nt))
+            go(std::integral_constant<int, R>{}, t512, cols_c);
+        else
+            go(std::integral_constant<int, 2>{}, t512, cols_c);
+    };
     if (nt > 512) {  // 1024 threads leave no registers for a second column's x
         go(std::integral_constant<int, 1>{}, std::integral_constant<int, kMaxThreads>{}, std::integral_constant<int, 1>{});
     } else {
         const int t1 = (a.out_len + a.slots * 2 - 1) / (a.slots * 2);
         switch (kq_columns(a.k, 4, t1, cu_count() * std::max(1, 1024 / nt) / 2)) {
         case 1: go(rows, t512, std::integral_constant<int, 1>{}); break;
-        case 2: go(std::integral_constant<int, 2>{}, t512, std::integral_constant<int, 2>{}); break;
-        case 3: go(std::integral_constant<int, 2>{}, t512, std::integral_constant<int, 3>{}); break;
-        default: go(std::integral_constant<int, 2>{}, t512, std::integral_constant<int, 4>{}); break;
+        case 2: cols(std::integral_constant<int, 2>{}); break;
+        case 3: cols(std::integral_constant<int, 3>{}); break;
+        default: cols(std::integral_constant<int, 4>{}); break;
         }
     }
     return check_launch("kq_gemv_kernel");
