@@ -462,14 +462,15 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
 // unnormalised output, max and sum go to `part`; attn_combine_kernel merges
 // the splits of each (b, head) and applies the sigmoid output gate.
 // A workgroup's keys are a serial chain (scores, softmax, P V), so a context of
-// up to kShortCtx keys takes more and shorter ones; the merge of the splits is
-// serial too, which is what bounds their number.  A sequence's splits follow
-// from its own length, so its result does not depend on the batch it is in.
-// One sequence of 300 keys, 4 kv heads: 17.7 -> 10.6 us; 48 sequences of 20000
-// keys in all: 33.5 -> 23.1 us.
+// up to kShortCtx keys takes more and shorter ones (one sequence of 300 keys, 4
+// kv heads: 17.7 -> 10.6 us).  Longer contexts fill the chip by themselves and
+// pay a workgroup's fixed cost per 64 keys (64 sequences of 16..2048 keys,
+// splits of 64 throughout: 2.95 against 2.81 ms per step of 24 layers).  A
+// sequence's splits follow from its own length, so its result does not depend
+// on the batch it is in.
 constexpr int kDecKeys = 256;
 constexpr int kDecKeysShort = 64;
-constexpr int kShortCtx = 2048;
+constexpr int kShortCtx = 512;
 __host__ __device__ constexpr int dec_keys(int len) { return len <= kShortCtx ? kDecKeysShort : kDecKeys; }
 // Splits that sequences of up to max_len keys can have.
 constexpr size_t dec_splits(size_t max_len) {

@@ -235,7 +235,7 @@ def test_stack_kv_page_pool(gpu):
 
 
 def test_stack_decode_split_lengths(gpu):
-    """Contexts of up to 2048 keys are decoded in splits of 64, longer ones in
+    """Contexts of up to 512 keys are decoded in splits of 64, longer ones in
     splits of 256.  One decode step after a prefill of n tokens gives the
     logits of a prefill of n + 1 (attention only: no bf16, so only summation
     orders and the few int8 roundings they flip differ), and a sequence's
@@ -244,7 +244,7 @@ def test_stack_decode_split_lengths(gpu):
     card = Card(n_layer=1, n_embd=256, n_ff=512, n_vocab=512, full_attention_interval=1, n_head=2, n_head_kv=1,
                 n_rot=64, ssm_n_k_heads=1, ssm_n_v_heads=2, eps=1e-6, rope_base=1e7)
     rng = np.random.default_rng(12)
-    prompts = [list(rng.integers(0, card.n_vocab, n)) for n in (2046, 62, 63, 64, 2047, 2048, 127, 2303, 1)]
+    prompts = [list(rng.integers(0, card.n_vocab, n)) for n in (510, 62, 63, 64, 511, 512, 127, 2303, 1)]
     feed = [[int(rng.integers(0, card.n_vocab)) for _ in prompts]]
     size = dict(max_seqs=len(prompts), max_tokens=12000, max_ctx=2400)
     dec, _ = gpu_run(card, prompts, feed, **size)
