@@ -452,7 +452,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
 
 
 // Decode attention, split over the context (flash-decoding): workgroup
-// (sequence b, kv head, split sp) takes keys sp*keys .. +keys of b (dec_keys)
+// (sequence b, kv head, split sp) takes keys sp*kDecKeys .. +kDecKeys of b
 // for all G = nh/nkv query heads of that kv head, so each K and V row is
 // read once per step.  Scores: 16 lanes per key (8 dims each, G dot
 // products, DPP row sums), 4 keys per wavefront per step, into LDS; per-head
@@ -461,24 +461,14 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
 // LDS.  The split's
 // unnormalised output, max and sum go to `part`; attn_combine_kernel merges
 // the splits of each (b, head) and applies the sigmoid output gate.
-// A workgroup's keys are a serial chain (scores, softmax, P V), so a context of
-// up to kShortCtx keys takes more and shorter ones (one sequence of 300 keys, 4
-// kv heads: 17.7 -> 10.6 us).  Longer contexts fill the chip by themselves and
-// pay a workgroup's fixed cost per 64 keys (64 sequences of 16..2048 keys,
-// splits of 64 throughout: 2.95 against 2.81 ms per step of 24 layers).  A
-// sequence's splits follow from its own length, so its result does not depend
-// on the batch it is in.
+// Every context is split alike, so a sequence's result does not depend on the
+// batch it is in.  Splits of 64 keys for contexts of up to 512 were faster for
+// one sequence (300 keys, 4 kv heads: 17.9 -> 10.7 us) and slower for batches,
+// whose workgroups fill the chip and pay their fixed cost four times as often
+// (64 sequences of 500 keys 29.1 -> 31.2, 256 of 500 94 -> 111, 48 of 40..790
+// keys 35.1 -> 45.5 us).
 constexpr int kDecKeys = 256;
-constexpr int kDecKeysShort = 64;
-constexpr int kShortCtx = 512;
-__host__ __device__ constexpr int dec_keys(int len) { return len <= kShortCtx ? kDecKeysShort : kDecKeys; }
-// Splits that sequences of up to max_len keys can have.
-constexpr size_t dec_splits(size_t max_len) {
-    const size_t s = max_len < kShortCtx ? max_len : kShortCtx;
-    const size_t a = (s + kDecKeysShort - 1) / kDecKeysShort, b = (max_len + kDecKeys - 1) / kDecKeys;
-    return a > b ? a : b;
-}
-constexpr int kMaxSplits = 128;  // of a context that the cache can hold (the merge has a thread for each)
+constexpr int kMaxSplits = 128;  // the merge has a thread for each (a context of 32768 keys)
 constexpr int kPartStride = kHd + 4;  // floats per (b, head, split) record: o[128], m, l
 
 template <int G>
@@ -490,11 +480,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G <= 4 ? 5 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int sp = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
     const int L = a.lens[b];
-    const int keys = dec_keys(L);
-    const int j0 = sp * keys;
+    const int j0 = sp * kDecKeys;
     if (j0 >= L) return;  // whole workgroup
-    const int n = min(keys, L - j0);
-    if (tid < keys / kPage && j0 + tid * kPage < L) prow[tid] = kv_row(a.pages, a.maxp, b, j0 + tid * kPage);
+    const int n = min(kDecKeys, L - j0);
+    if (tid < kDecKeys / kPage && j0 + tid * kPage < L) prow[tid] = kv_row(a.pages, a.maxp, b, j0 + tid * kPage);
     __syncthreads();
     const int g4 = lane >> 4, gl = lane & 15;
     float4 q[G][2];
@@ -507,16 +496,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G <= 4 ? 5 
     // scores: wave w, step it -> key w*kWK + 4*it + g4 (a wave's keys lie in
     // one page); rows past the split are clamped to its last key, so the
     // loads carry no branches, and their scores are not stored
-    const int kWK = keys / 4;  // keys per wavefront
-    static_assert(kPage % (kDecKeys / 4) == 0 && kDecKeys % kDecKeysShort == 0 && kDecKeysShort % kPage == 0,
-                  "a wavefront's keys lie in one page");
+    constexpr int kWK = kDecKeys / 4;  // keys per wavefront
+    static_assert(kPage % kWK == 0, "a wavefront's keys lie in one page");
     const int wkeys = min(kWK, n - wave * kWK);  // keys of this wave (<= 0: none)
     const long long wrow = wkeys > 0 ? prow[wave * kWK / kPage] + wave * kWK % kPage : 0;
     // kB key rows' loads are issued together before their dot products: the
     // conditional score store splits an iteration into several basic blocks,
     // so the compiler would not hoist the next key's loads across it
     constexpr int kB = 4;
-    static_assert(kDecKeysShort / 16 % kB == 0, "whole load batches");
+    static_assert((kWK / 4) % kB == 0, "whole load batches");
     for (int it0 = 0; it0 < (wkeys > 0 ? kWK / 4 : 0); it0 += kB) {
         float4 k0[kB], k1[kB];
 #pragma unroll
@@ -611,7 +599,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G <= 4 ? 5 
 // times sigmoid(gate) (qwen35.rs:1205-1210).  One 128-thread workgroup per (b, head).
 __global__ __launch_bounds__(128) void attn_combine_kernel(AttnArgs a, const float *part, int nsplit) {
     const int b = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-    const int keys = dec_keys(a.lens[b]), ns = (a.lens[b] + keys - 1) / keys;
+    const int ns = (a.lens[b] + kDecKeys - 1) / kDecKeys;
     const float *rec = part + (static_cast<long long>(b) * a.nh + h) * nsplit * kPartStride;
     // the splits' maxima and sums together, one a thread, then the outputs
     // with their loads independent of each other
@@ -922,7 +910,7 @@ int attn_prefill(const float *q, const float *gate, const float *kc, const float
 }
 
 size_t attn_decode_ws_bytes(size_t B, int nh, size_t max_ctx) {
-    return B * static_cast<size_t>(nh) * dec_splits(max_ctx) * kPartStride * sizeof(float);
+    return B * static_cast<size_t>(nh) * ((max_ctx + kDecKeys - 1) / kDecKeys) * kPartStride * sizeof(float);
 }
 
 int attn_decode(const float *q, const float *gate, const float *kc, const float *vc, const int32_t *pages, int maxp,
@@ -930,7 +918,7 @@ int attn_decode(const float *q, const float *gate, const float *kc, const float 
     const int G = nh / nkv;
     if (G < 1 || G > 8 || nh % nkv) return fail(OURO_ERR_SHAPE, "attn_decode: %d heads over %d kv heads", nh, nkv);
     if (max_len < 1 || !B) return OURO_OK;
-    const int nsplit = static_cast<int>(dec_splits(max_len));
+    const int nsplit = (max_len + kDecKeys - 1) / kDecKeys;
     if (nsplit > kMaxSplits) return fail(OURO_ERR_SHAPE, "attn_decode: context %d", max_len);
     AttnArgs a{q, gate, kc, vc, pages, nullptr, lens, nullptr, nullptr, out, nh, nkv, maxp,
                1.0f / sqrtf(static_cast<float>(kHd))};

@@ -235,20 +235,22 @@ def test_stack_kv_page_pool(gpu):
 
 
 def test_stack_decode_split_lengths(gpu):
-    """Contexts of up to 512 keys are decoded in splits of 64, longer ones in
-    splits of 256.  One decode step after a prefill of n tokens gives the
-    logits of a prefill of n + 1 (attention only: no bf16, so only summation
-    orders and the few int8 roundings they flip differ), and a sequence's
-    logits do not depend on the others in the batch, long or short, bit for
-    bit."""
+    """Keys are decoded in splits of 256 (test_attn_decode.py holds the splits
+    and their merge to float64).  Here the stack hands each sequence's length
+    and pages over: one decode step after a prefill of n tokens gives the
+    logits of a prefill of n + 1, judged for each sequence by itself
+    (attention only: no bf16, so only summation orders and the few int8
+    roundings they flip differ), and every sequence, long or short, has the
+    same logits alone as in the batch, bit for bit."""
     card = Card(n_layer=1, n_embd=256, n_ff=512, n_vocab=512, full_attention_interval=1, n_head=2, n_head_kv=1,
                 n_rot=64, ssm_n_k_heads=1, ssm_n_v_heads=2, eps=1e-6, rope_base=1e7)
     rng = np.random.default_rng(12)
-    prompts = [list(rng.integers(0, card.n_vocab, n)) for n in (510, 62, 63, 64, 511, 512, 127, 2303, 1)]
+    prompts = [list(rng.integers(0, card.n_vocab, n)) for n in (510, 62, 63, 64, 511, 512, 127, 2303, 1, 255, 256)]
     feed = [[int(rng.integers(0, card.n_vocab)) for _ in prompts]]
     size = dict(max_seqs=len(prompts), max_tokens=12000, max_ctx=2400)
     dec, _ = gpu_run(card, prompts, feed, **size)
     pre, _ = gpu_run(card, [p + [f] for p, f in zip(prompts, feed[0])], [], **size)
-    assert rel(dec[1], pre[0]) < TOL_BF16
-    short, _ = gpu_run(card, prompts[1:4], [feed[0][1:4]], **size)
-    assert np.array_equal(short[1], dec[1][1:4])
+    for i in range(len(prompts)):
+        assert rel(dec[1][i], pre[0][i]) < TOL_BF16, len(prompts[i])
+        alone, _ = gpu_run(card, prompts[i:i + 1], [feed[0][i:i + 1]], **size)
+        assert np.array_equal(alone[1][0], dec[1][i]), len(prompts[i])
