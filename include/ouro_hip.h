@@ -11,7 +11,8 @@
  * synchronise of that stream) and kept until ouro_stream_destroy() of the
  * stream or ouro_shutdown():
  *   - ouro_matvec_q / ouro_matmul_q on the 2-bit kinds (the int8
- *     activations of x);
+ *     activations of x; not for one column of a tiled I2 payload of limited
+ *     size, which is quantised inside the product);
  *   - ouro_matvec_q on a raw TL1 or TQ1_0 payload of 8192 rows or more
  *     (k == 1): the lookup kernels' per-block partial sums;
  *   - ouro_matmul_q on a raw TL1 payload for k >= 2 columns: x as int8
@@ -266,7 +267,9 @@ int ouro_gemm_i2_mfma(const uint8_t *w_mfma, size_t out_len, size_t in_len,
  *                     in_len % 256 == 0, in_len <= 32768)
  *   OURO_KIND_I2    - tiled I2 + scale
  *   For both ternary 2-bit kinds x is quantised per call (quantize_row_i8_s,
- *   above) into the library workspace.  TL1 and TQ1_0 payloads of 8192 rows
+ *   above): one column of a tiled I2 payload of limited size inside the
+ *   product, without scratch; all else into the library workspace.  y may
+ *   overlap x for these two kinds, not for the others.  TL1 and TQ1_0 payloads of 8192 rows
  *   or more run the table-lookup kernels, whose per-block partial sums also
  *   live in the library workspace (per stream; ouro_matvec_q_noalloc or a
  *   weight handle keeps these calls allocation-free).

@@ -170,6 +170,12 @@ __global__ __launch_bounds__(64 * kWaves) void tq1_kernel(MvArgs a) {
     wave_store<NC>(acc, a, row, c0, lane);
 }
 
+// x[0 .. nx) and y[0 .. ny) share memory
+bool overlap(const float *x, size_t nx, const float *y, size_t ny) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(y);
+    return a < b + ny * sizeof(float) && b < a + nx * sizeof(float);
+}
+
 int launch_mv(int kind, const MvArgs &a, hipStream_t s) {
     const int nc = a.k >= 8 ? 8 : (a.k >= 4 ? 4 : (a.k >= 2 ? 2 : 1));
     dim3 grid((a.out_len + kWaves - 1) / kWaves, (a.k + nc - 1) / nc), block(64 * kWaves);
@@ -265,7 +271,9 @@ int matmul_q(const void *payload, int kind, size_t out_len, size_t in_len, const
     case OURO_KIND_I2_S: {
         const size_t tb = i2_tiled_bytes(out_len, in_len);
         if (!tb) return fail(OURO_ERR_SHAPE, "matvec_q I2: in_len %zu not a multiple of 256", in_len);
-        if (kind == OURO_KIND_I2 && k == 1 && i2_matvec_f32_pays(out_len, in_len)) {  // one launch, no scratch
+        // one launch, no scratch; y over x (in place) takes the copy of x below, which
+        // is whole before the first y is written
+        if (kind == OURO_KIND_I2 && k == 1 && i2_matvec_f32_pays(out_len, in_len) && !overlap(x, in_len, y, out_len)) {
             const uint8_t *w = static_cast<const uint8_t *>(payload);
             return i2_matvec_f32(w, out_len, in_len, reinterpret_cast<const float *>(w + tb), x, y, stream);
         }

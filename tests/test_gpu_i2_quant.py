@@ -61,3 +61,28 @@ def test_matvec_rounds_x_itself(gpu, out_len, in_len):
         call("ouro_act_quant_i8", xd.ptr, DT_F32, 1, in_len, q.ptr, s.ptr, None)
         call("ouro_gemm_i2", payload, out_len, in_len, scale, q.ptr, s.ptr, 1, y2.ptr, None, None)
         assert np.array_equal(y.download().view(np.uint32), y2.download().view(np.uint32))
+
+
+@pytest.mark.parametrize("out_len,in_len", [(2560, 2560), (8192, 8192), (1000, 4096), (6000, 1024)])
+@pytest.mark.parametrize("shift", [0, 40, -40])
+def test_matvec_in_place(gpu, out_len, in_len, shift):
+    """y over x, whole or in part, by a handle, a payload and without allocation: the bits of y elsewhere."""
+    rng = np.random.default_rng(out_len)
+    w = rng.integers(-1, 2, size=(out_len, in_len)).astype(np.int8)
+    h = ops.Weight(QuantKind.I2, i2_pack(w), out_len, in_len, w_scale=0.7)
+    payload = _lib.lib().ouro_weight_payload(h.handle)
+    x = inputs(rng, 2, in_len)[1]
+    xd, y = DeviceBuffer.from_host(x), DeviceBuffer((out_len,), np.float32)
+    call("ouro_weight_matvec", h.handle, xd.ptr, y.ptr, None)
+    want = y.download()
+    at, n = 64, 128 + max(out_len, in_len)
+    host = np.zeros(n, np.float32)
+    host[at:at + in_len] = x
+    buf = DeviceBuffer((n,), np.float32)
+    xp, yp = buf.ptr + 4 * at, buf.ptr + 4 * (at + shift)
+    for fn, *a in (("ouro_weight_matvec", h.handle), ("ouro_matvec_q", payload, int(QuantKind.I2), out_len, in_len),
+                   ("ouro_matvec_q_noalloc", payload, int(QuantKind.I2), out_len, in_len)):
+        buf.upload(host)
+        call(fn, *a, xp, yp, None)
+        got = buf.download()[at + shift:at + shift + out_len]
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), fn
