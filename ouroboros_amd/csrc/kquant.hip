@@ -50,6 +50,7 @@
 #include "common.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -1584,9 +1585,17 @@ int launch_mfma(const char *what, Pick pick, const KqArgs &a, int tiles, int cap
                          : nc == 3 ? pick(std::integral_constant<int, 3>{})
                                    : pick(std::integral_constant<int, 4>{});
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return fail(OURO_ERR_HIP, "%s: %zu B of LDS refused: %s", what, lds, hipGetErrorString(e));
+        // the opt-in, once per kernel and device and always to the largest
+        // size, so that threads with different rows never lower each other's
+        static std::atomic<uint64_t> set[4];
+        const int dev = current_device();
+        const uint64_t bit = dev >= 0 && dev < 64 ? uint64_t(1) << dev : 0;
+        if (!(set[nc - 1].load(std::memory_order_acquire) & bit)) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsMax));
+            if (e != hipSuccess) return fail(OURO_ERR_HIP, "%s: %zu B of LDS refused: %s", what, kLdsMax, hipGetErrorString(e));
+            set[nc - 1].fetch_or(bit, std::memory_order_release);
+        }
     }
     if (nc > 1) cap = std::min(cap, static_cast<int>(kLdsMax / lds));  // no more than fit: each converts x anew
     const dim3 grid(std::min(tiles, cu_count() * cap), (a.k + nc - 1) / nc);

@@ -7,13 +7,14 @@ rel 1e-3 for matmul, ops.rs:720-750), and per row
 layer 6912x2560 and the lm_head probe 248320x5120; misaligned payloads; the
 >512-task and >1024-task rows; each tiling of the matrix-core kernels."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
 
 from ouroboros_amd import ops
 from ouroboros_amd._lib import OuroError, call
-from ouroboros_amd.device import DeviceBuffer
+from ouroboros_amd.device import DeviceBuffer, Stream, synchronize
 from ouroboros_amd.quant import QuantKind
 
 pytestmark = pytest.mark.gpu
@@ -274,3 +275,35 @@ def test_kquant_column_groups(gpu, kind, out_len, in_len, offset):
         got = y.download().reshape(11, out_len)
         assert np.array_equal(got[:k], one[:k]), k
         assert np.isnan(got[k:]).all()
+
+
+def test_two_threads_different_rows(gpu):
+    """Two host threads in one kernel with row lengths that take different
+    amounts of LDS past 64 KiB: the opt-in of one never lowers the other's."""
+    kind, out_len, k = QuantKind.Q8_0, 8200, 4
+    rng = np.random.default_rng(3)
+    jobs = []
+    for in_len in (8192, 5120):  # about 142 and 96 KiB
+        buf = DeviceBuffer.from_host(kq_payload(rng, kind, out_len, in_len))
+        x = DeviceBuffer.from_host(rng.standard_normal((k, in_len)).astype(np.float32))
+        y = DeviceBuffer((k, out_len), np.float32)
+        call("ouro_matmul_q", buf.ptr, int(kind), out_len, in_len, x.ptr, k, y.ptr, None)
+        jobs.append((buf, in_len, x, y, y.download(), Stream()))
+    errors = []
+
+    def work(buf, in_len, x, y, want, stream):
+        try:
+            for _ in range(200):
+                call("ouro_matmul_q", buf.ptr, int(kind), out_len, in_len, x.ptr, k, y.ptr, stream.handle)
+        except Exception as e:  # handed to the test's own thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    synchronize()
+    assert not errors
+    for _, _, _, y, want, _ in jobs:
+        assert np.array_equal(y.download(), want)
