@@ -438,16 +438,16 @@ constexpr int kBatch1 = 64;
 __device__ __forceinline__ void vm_drain() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
 template <int R>
-__device__ __forceinline__ void stash(float *red, const float (&v)[R], int b) {  // b: tile of the batch, column by column
-    const int t = threadIdx.x, nt = blockDim.x;
+__device__ __forceinline__ void stash(float *red, const float (&v)[R], int b, int nt) {  // b: tile of the batch, column by column
+    const int t = threadIdx.x;
 #pragma unroll
     for (int r = 0; r < R; ++r) red[(b * R + r) * nt + t] = v[r];
 }
 
 // Rows of the nb tiles tile0, tile0 + g, ... of a batch.
 template <int R, int NC>
-__device__ __forceinline__ void flush(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0) {
-    const int t = threadIdx.x, nt = blockDim.x;
+__device__ __forceinline__ void flush(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0, int nt) {
+    const int t = threadIdx.x;
     const int rows_per_tile = a.slots * R;
     const int wave = t >> 6, lane = t & 63, nwaves = nt >> 6;
     __syncthreads();
@@ -510,8 +510,8 @@ __device__ __forceinline__ float row_totals_f(float (&v)[R]) {
 // slots == 1: the wavefront's totals of tile b's R rows into LDS (lanes past
 // the task set add 0).
 template <int R>
-__device__ __forceinline__ void stash1(float *red, float (&v)[R], int b, bool live) {
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nwaves = blockDim.x >> 6;
+__device__ __forceinline__ void stash1(float *red, float (&v)[R], int b, bool live, int nt) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nwaves = nt >> 6;
     if (!live) {
 #pragma unroll
         for (int r = 0; r < R; ++r) v[r] = 0.f;
@@ -522,10 +522,10 @@ __device__ __forceinline__ void stash1(float *red, float (&v)[R], int b, bool li
 }
 
 template <int R, int NC>
-__device__ __forceinline__ void flush1(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0) {
-    const int t = threadIdx.x, nwaves = blockDim.x >> 6;
+__device__ __forceinline__ void flush1(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0, int nt) {
+    const int t = threadIdx.x, nwaves = nt >> 6;
     __syncthreads();
-    for (int o = t; o < nb * NC * R; o += blockDim.x) {
+    for (int o = t; o < nb * NC * R; o += nt) {
         const int b = o / R, r = o - b * R, col = c0 + b % NC;
         float acc = 0.f;
         for (int w = 0; w < nwaves; ++w) acc += red[(b * R + r) * nwaves + w];
@@ -552,6 +552,10 @@ void kq_gemv_kernel(KqArgs a) {
     using F = Fmt<KIND>;
     extern __shared__ float red[];  // slots == 1: [kBatch1][R][wavefronts], else [kBatch][R][blockDim.x]
     const int t = threadIdx.x;
+    // once, into a scalar register: inside the tile loop the compiler fetched it
+    // by a vector load, whose wait also held the next tile's loads (20000x20480
+    // Q6_K 89 -> 76 us)
+    const int nt = __builtin_amdgcn_readfirstlane(static_cast<int>(blockDim.x));
     const int slot = min(t / a.tpr, a.slots - 1);
     const int task = min(t - slot * a.tpr, a.tpr - 1);
     const int blk = task / F::TPB, u = task % F::TPB;
@@ -596,14 +600,14 @@ void kq_gemv_kernel(KqArgs a) {
         }
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            if (one) stash1<R>(red, v[c], nb * NC + c, live);
-            else stash<R>(red, v[c], nb * NC + c);
+            if (one) stash1<R>(red, v[c], nb * NC + c, live, nt);
+            else stash<R>(red, v[c], nb * NC + c, nt);
         }
         ++nb;
         tile += g;
         if (nb == batch || tile >= a.tiles) {  // uniform over the workgroup
-            if (one) flush1<R, NC>(a, red, nb, tile0, g, c0);
-            else flush<R, NC>(a, red, nb, tile0, g, c0);
+            if (one) flush1<R, NC>(a, red, nb, tile0, g, c0, nt);
+            else flush<R, NC>(a, red, nb, tile0, g, c0, nt);
             nb = 0;
             tile0 = tile;
         }
