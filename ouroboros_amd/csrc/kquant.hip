@@ -24,9 +24,10 @@
 // quarter-width dot steps.
 //
 // Several columns (matmul_q) are taken up to four at a time by every kernel
-// here: the codes are read and decoded once for the group, and each column's
-// products, scales and sums are those of a single column, so a column of
-// matmul_q is matvec_q of it bit for bit (kq_columns).
+// here (rows of several task sets a workgroup, below, one by one): the codes are
+// read and decoded once for the group, and each column's products, scales and
+// sums are those of a single column, so a column of matmul_q is matvec_q of it
+// bit for bit (kq_columns).
 //
 // Mapping.  A thread owns one task position of a row (k-stationary): its 32 x
 // values and their run sums stay in registers while the workgroup walks row
@@ -422,13 +423,13 @@ __device__ __forceinline__ void load_x(const float *xc, int blk, int u, XRun &xa
 // memory counter covers loads and stores in issue order) before it reuses the
 // store's registers.
 //
-// Several task sets per workgroup (slots > 1): each thread's sum of each row
+// Several task sets per workgroup (slots > 1, one column): each thread's sum of each row
 // of a batch of up to kBatch tiles, red[(b R + r) nt + t]; one wavefront per
 // row adds a row's task sums.
-constexpr int kBatch = 4;  // tiles times columns
+constexpr int kBatch = 4;
 // One task set per workgroup (slots == 1): each wavefront adds its lanes'
 // sums in registers and keeps one value per row, red[(b R + r) nwaves +
-// wave], for a batch of up to kBatch1 tiles.
+// wave], for a batch of up to kBatch1 tiles times columns.
 constexpr int kBatch1 = 64;
 
 // s_waitcnt vmcnt(0) (gfx9 encoding: expcnt and lgkmcnt left at their
@@ -438,29 +439,29 @@ constexpr int kBatch1 = 64;
 __device__ __forceinline__ void vm_drain() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
 template <int R>
-__device__ __forceinline__ void stash(float *red, const float (&v)[R], int b, int nt) {  // b: tile of the batch, column by column
+__device__ __forceinline__ void stash(float *red, const float (&v)[R], int b, int nt) {
     const int t = threadIdx.x;
 #pragma unroll
     for (int r = 0; r < R; ++r) red[(b * R + r) * nt + t] = v[r];
 }
 
 // Rows of the nb tiles tile0, tile0 + g, ... of a batch.
-template <int R, int NC>
-__device__ __forceinline__ void flush(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0, int nt) {
+template <int R>
+__device__ __forceinline__ void flush(const KqArgs &a, const float *red, int nb, int tile0, int g, int col, int nt) {
     const int t = threadIdx.x;
     const int rows_per_tile = a.slots * R;
     const int wave = t >> 6, lane = t & 63, nwaves = nt >> 6;
     __syncthreads();
-    for (int o = wave; o < nb * NC * rows_per_tile; o += nwaves) {
-        const int b = o / rows_per_tile, ob = o - b * rows_per_tile, col = c0 + b % NC;
+    for (int o = wave; o < nb * rows_per_tile; o += nwaves) {
+        const int b = o / rows_per_tile, ob = o - b * rows_per_tile;
         const int s = ob / R, r = ob - s * R;
         const float *src = red + (b * R + r) * nt + s * a.tpr;
         float acc = 0.f;
         for (int i = lane; i < a.tpr; i += 64) acc += src[i];
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) acc += xor_shfl(acc, off);
-        const int row = (tile0 + b / NC * g) * rows_per_tile + ob;
-        if (lane == 0 && row < a.out_len && col < a.k) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
+        const int row = (tile0 + b * g) * rows_per_tile + ob;
+        if (lane == 0 && row < a.out_len) a.y[static_cast<long long>(col) * a.out_len + row] = acc;
     }
     __syncthreads();
     vm_drain();
@@ -521,6 +522,7 @@ __device__ __forceinline__ void stash1(float *red, float (&v)[R], int b, bool li
     if (lane % span == span - 1) red[(b * R + lane / span) * nwaves + wave] = s;
 }
 
+// b: tile of the batch, column by column
 template <int R, int NC>
 __device__ __forceinline__ void flush1(const KqArgs &a, const float *red, int nb, int tile0, int g, int c0, int nt) {
     const int t = threadIdx.x, nwaves = nt >> 6;
@@ -540,17 +542,18 @@ __device__ __forceinline__ void flush1(const KqArgs &a, const float *red, int nb
 // next tile are issued before the current one is summed (two register sets).
 // Lanes past the last slot (padding to a whole wavefront) run a clamped copy
 // of a real task whose sums are never read, so no load sits behind a branch.
-// Wavefronts per SIMD the register allocation is held to: Q3_K fits 4
-// (136 -> 128 VGPRs, no spill); the other kinds are left as the compiler
-// allocates them (4 waves already; Q8_0 held to 5 ran 10 % slower, the
-// others spill when pressed).
-template <int KIND, int NC> constexpr int kWavesPerSimd = KIND == OURO_KIND_Q3K && NC == 1 ? 4 : 1;
+// Wavefronts per SIMD the register allocation is held to: Q3_K and Q6_K fit 4
+// (136 and 130 -> 128 VGPRs, no spill; Q6_K 248320x1280 92 -> 74 us); the
+// other kinds are left as the compiler allocates them (Q8_0 held to 5 ran 10 %
+// slower, the others spill when pressed).
+template <int KIND, int NC>
+constexpr int kWavesPerSimd = (KIND == OURO_KIND_Q3K || KIND == OURO_KIND_Q6K) && NC == 1 ? 4 : 1;
 
 template <int KIND, int R, bool AL16, bool PH, int MAXT, int NC>
 __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<KIND, NC>)))
 void kq_gemv_kernel(KqArgs a) {
     using F = Fmt<KIND>;
-    extern __shared__ float red[];  // slots == 1: [kBatch1][R][wavefronts], else [kBatch][R][blockDim.x]
+    extern __shared__ float red[];  // slots == 1: [kBatch1][R][wavefronts], else (NC == 1) [kBatch][R][blockDim.x]
     const int t = threadIdx.x;
     // once, into a scalar register: inside the tile loop the compiler fetched it
     // by a vector load, whose wait also held the next tile's loads (20000x20480
@@ -585,10 +588,9 @@ void kq_gemv_kernel(KqArgs a) {
     if (tile >= a.tiles) return;
     int tile0 = tile, nb = 0;  // the batch's first tile and its tiles so far
     // sum one tile into the batch; a full batch, or the last tile, is added up
-    const bool one = a.slots == 1;          // uniform
+    const bool one = NC > 1 || a.slots == 1;  // uniform
     const bool live = t < a.tpr * a.slots;  // not a padding lane
-    constexpr int kB1 = kBatch1 / NC, kB = kBatch / NC;
-    const int batch = one ? kB1 : kB;
+    const int batch = one ? kBatch1 / NC : kBatch;
     auto sum = [&](const typename F::Raw(&raw)[R]) {
         float v[NC][R];
 #pragma unroll
@@ -601,13 +603,13 @@ void kq_gemv_kernel(KqArgs a) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             if (one) stash1<R>(red, v[c], nb * NC + c, live, nt);
-            else stash<R>(red, v[c], nb * NC + c, nt);
+            else stash<R>(red, v[c], nb, nt);
         }
         ++nb;
         tile += g;
         if (nb == batch || tile >= a.tiles) {  // uniform over the workgroup
             if (one) flush1<R, NC>(a, red, nb, tile0, g, c0, nt);
-            else flush<R, NC>(a, red, nb, tile0, g, c0, nt);
+            else flush<R>(a, red, nb, tile0, g, c0, nt);
             nb = 0;
             tile0 = tile;
         }
@@ -1500,10 +1502,22 @@ int cu_count() {
 }
 
 // Threads a CU of the task kernel's grid.  Each workgroup converts x once and
-// walks its tiles; what does not fit on the chip at once converts it for
-// nothing (4096x14336 Q6_K, one column: 2048 threads a CU 16.3, 1024 13.2, 512
-// 12.8 us; six columns, three at a time, two rows a tile, 77 / 56 / 46 us).
-constexpr int kTaskThreads = 512;
+// walks its tiles.  One task set a workgroup (slots == 1): two wavefronts a SIMD
+// keep enough loads in flight, and more convert x again (512 against 2048
+// threads, us, cold: Q6_K 4096x14336 12.6 / 17.6, 8192x8192 off a dword 14.1 /
+// 19.5, 50000x14336 107 / 110, 20000x20480 66.7 / 75.8, 248320x2048 79.7 / 86.8).
+// Several: a batch's sums stop its workgroup every kBatch tiles, so as many as
+// the registers let a CU hold work in turn (three wavefronts a SIMD for Q4_K and
+// Q5_K, four for the others; 512 / 768 / 1024 threads: Q6_K 60000x768 24.5 / 19.9 /
+// 19.2, 120000x1280 47.0 / 45.9 / 39.6, 200000x3072 154 / 119 / 119; Q4_K there 26.2 /
+// 19.3 / 23.5, 42.3 / 34.7 / 42.6, 132 / 98 / 111).  A Q4_K row of up to 640 threads
+// fits twice (40000x20480 109 -> 98).
+template <int KIND>
+constexpr int task_threads(int slots, int nt) {
+    constexpr bool q4 = KIND == OURO_KIND_Q4K, q5 = KIND == OURO_KIND_Q5K;
+    if (slots > 1) return q4 || q5 ? 768 : 1024;
+    return q4 && nt > 512 ? 1280 : 512;
+}
 
 // Launch shape for rows of tpr tasks: slots side by side in a workgroup of
 // nt threads (up to 256 threads, the most rows side by side with the fewest
@@ -1674,18 +1688,19 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
     }
     a.slots = pl.slots;
     const int nt = pl.nt;
+    const int wgs = cu_count() * std::max(1, task_threads<KIND>(pl.slots, nt) / nt);
     auto go = [&](auto rows_c, auto maxt_c, auto cols_c) {
         constexpr int R = decltype(rows_c)::value, MAXT = decltype(maxt_c)::value, NC = decltype(cols_c)::value;
         a.tiles = (a.out_len + a.slots * R - 1) / (a.slots * R);
-        const int grid_x = std::min(a.tiles, cu_count() * std::max(1, kTaskThreads / nt));
         const size_t lds = (a.slots == 1 ? static_cast<size_t>(kBatch1 / NC * NC) * R * (nt / 64)
-                                         : static_cast<size_t>(kBatch / NC * NC) * R * nt) * sizeof(float);
-        dim3 grid(grid_x, (a.k + NC - 1) / NC);
+                                         : static_cast<size_t>(kBatch) * R * nt) * sizeof(float);
+        dim3 grid(std::min(a.tiles, wgs), (a.k + NC - 1) / NC);
         if (al16) hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, true, false, MAXT, NC>), grid, dim3(nt), lds, s, a);
         else if (ph) hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, true, MAXT, NC>), grid, dim3(nt), lds, s, a);
         else hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, false, MAXT, NC>), grid, dim3(nt), lds, s, a);
     };
     constexpr std::integral_constant<int, kRows<KIND>> rows{};
+    constexpr std::integral_constant<int, 1> c1{};
     constexpr std::integral_constant<int, 512> t512{};
     // Several columns: four rows a tile where that still gives every workgroup
     // two tiles, else two (three columns of Q6_K, R = 2 / 4: 32768x1792 24.7 /
@@ -1693,17 +1708,19 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
     auto cols = [&](auto cols_c) {
         // four columns of Q3_K and Q5_K leave no registers for four rows
         constexpr int R = decltype(cols_c)::value == 4 && (KIND == OURO_KIND_Q3K || KIND == OURO_KIND_Q5K) ? 2 : 4;
-        if ((a.out_len + a.slots * 4 - 1) / (a.slots * 4) >= 2 * cu_count() * std::max(1, kTaskThreads / nt))
-            go(std::integral_constant<int, R>{}, t512, cols_c);
-        else
-            go(std::integral_constant<int, 2>{}, t512, cols_c);
+        if ((a.out_len + 3) / 4 >= 2 * wgs) go(std::integral_constant<int, R>{}, t512, cols_c);
+        else go(std::integral_constant<int, 2>{}, t512, cols_c);
     };
     if (nt > 512) {  // 1024 threads leave no registers for a second column's x
-        go(std::integral_constant<int, 1>{}, std::integral_constant<int, kMaxThreads>{}, std::integral_constant<int, 1>{});
+        go(c1, std::integral_constant<int, kMaxThreads>{}, c1);
+    } else if (a.slots > 1) {
+        // a column's sums cost more than the decode it would share (four columns,
+        // one by one / grouped: Q6_K 60000x768 58.9 / 89.9, 20000x512 20.9 / 32.2,
+        // 60000x3072 121 / 143 us)
+        go(rows, t512, c1);
     } else {
-        const int t1 = (a.out_len + a.slots * 2 - 1) / (a.slots * 2);
-        switch (kq_columns(a.k, 4, t1, cu_count() * std::max(1, 1024 / nt) / 2)) {
-        case 1: go(rows, t512, std::integral_constant<int, 1>{}); break;
+        switch (kq_columns(a.k, 4, (a.out_len + 1) / 2, cu_count() * std::max(1, 1024 / nt) / 2)) {
+        case 1: go(rows, t512, c1); break;
         case 2: cols(std::integral_constant<int, 2>{}); break;
         case 3: cols(std::integral_constant<int, 3>{}); break;
         default: cols(std::integral_constant<int, 4>{}); break;
