@@ -27,7 +27,7 @@
 // here (rows of several task sets a workgroup, below, one by one): the codes are
 // read and decoded once for the group, and each column's products, scales and
 // sums are those of a single column, so a column of matmul_q is matvec_q of it
-// bit for bit (kq_columns).
+// bit for bit (task_columns, mfma_columns).
 //
 // Mapping.  A thread owns one task position of a row (k-stationary): its 32 x
 // values and their run sums stay in registers while the workgroup walks row
@@ -1569,34 +1569,73 @@ int kq_tiling(int out_len, size_t lds, int steps, bool any_sh) {
     return 0;
 }
 
-// Columns a workgroup takes at once (1..4) for k of them: the least work, a
-// pass over the codes (load and decode) costing about one column's products
-// and conversion of x, among the counts that LDS holds (fit) and that leave
-// enough workgroups: tiles * column groups >= wgs.  Columns one by one then
-// overlap better (Q6_K 300x2560, 4 columns: 4.3 us, as one group 9.2).
-// Measured, one by one -> grouped: Q6_K 8192x8192 2 / 4 columns 24.8 / 45.3 ->
-// 16.9 / 25.2 us, 20000x3072 9 columns 77 -> 50; Q4_K there 13.0 / 22.6 ->
-// 13.5 / 22.1 and 45 -> 31 us.
-int kq_columns(int k, int fit, long long tiles, long long wgs) {
-    int best = 1, cost = 2 * k;
-    for (int nc = 2; nc <= std::min(4, fit); ++nc) {
-        const int groups = (k + nc - 1) / nc, c = groups * (1 + nc);
-        if (c < cost && tiles * groups >= wgs) best = nc, cost = c;
+// Columns a workgroup of the task kernel takes at once (1..4) for k of them,
+// where one row is its task set: the fewest products, decodes (two columns'
+// products a row) and conversions of x (eight rows' products a column) of a
+// workgroup, times the rounds that `wgs` of them at a time make of the launch.
+// rows(nc): rows a tile.  Over 1.7 thousand timings (all five kinds, 2048 to 16384
+// elements, 64 to 20000 rows, 2 to 16 columns) 1 % above the best of the four on
+// average; the rule before, which counted no rounds, 3 % with some short
+// matrices far off (five columns, us, one by one / that rule / this one: Q3_K
+// 200x16384 8.3 / 13.1 / 8.3, Q4_K 1000x5120 9.0 / 12.5 / 9.0).
+template <class Rows>
+int task_columns(int k, int out_len, int wgs, Rows rows) {
+    int best = 1;
+    long long least = 0;
+    for (int nc = 1; nc <= std::min(k, 4); ++nc) {
+        const int r = rows(nc), tiles = (out_len - 1) / r + 1, gx = std::min(tiles, wgs), groups = (k + nc - 1) / nc;
+        const long long rounds = (static_cast<long long>(gx) * groups + wgs - 1) / wgs;
+        const long long c = rounds * (static_cast<long long>((tiles - 1) / gx + 1) * r * (2 + nc) + 8 * nc);
+        if (nc == 1 || c < least) best = nc, least = c;
+    }
+    return best;
+}
+
+// The decode of a pass over the codes, in halves of a column's products.
+template <int KIND>
+constexpr int kDecode = KIND == OURO_KIND_Q4K ? 1 : KIND == OURO_KIND_Q3K || KIND == OURO_KIND_Q5K ? 2 : 6;
+
+// Columns a workgroup of a matrix-core kernel takes at once (1..4) for k of
+// them.  A group decodes once, but its planes take more LDS, so a CU holds
+// fewer workgroups and the launch more rounds of them.  Columns one by one
+// that fit in a single round stay so.  Else the least estimate: a CU's share
+// of the tiles at decode + 2 a column, and 8 a round of what the CUs hold
+// together; a group counts a twelfth more, and one that has a CU to itself is
+// left out where the CUs have fewer than three tiles for every two (its four
+// wavefronts keep too few loads in flight).  Constants fitted to 2.6 thousand
+// timings (all five kinds, 2560 to 14336 elements, 2048 to 40000 rows, 2 to 12
+// columns): 2.5 % above the best of the four on average, one by one 28 %, a
+// count of decodes and products alone 7 %, since it grouped short matrices
+// into more rounds (us, one by one / that count / this: Q4_K 3000x8192 five
+// columns 13.6 / 21.5 / 13.6, 4096x10240 eight 30.8 / 49.1 / 30.8, 8192x8192 two
+// 13.1 / 13.4 / 13.1; Q8_0 8192x12288 two 38.6 / 38.6 / 28.1; Q6_K 8192x8192 four
+// 45 / 25 / 25).
+int mfma_columns(int k, int decode, int tiles, int cap, size_t planes, size_t rest) {
+    const int cus = cu_count();
+    int best = 1;
+    long long least = 0;
+    for (int nc = 1; nc <= std::min(k, 4); ++nc) {
+        const size_t lds = nc * planes + rest;
+        if (nc > 1 && lds > kLdsMax) break;
+        const int groups = (k + nc - 1) / nc, per = std::max(1, std::min(cap, static_cast<int>(kLdsMax / lds)));
+        if (nc > 1 && per == 1 && 2LL * tiles < 3LL * cus) continue;
+        const long long n = static_cast<long long>(tiles) * groups, slots = static_cast<long long>(cus) * per;
+        long long c = 12 * ((n + cus - 1) / cus * (decode + 2 * nc) + (n + slots - 1) / slots * 8);
+        if (nc > 1) c += c / 12;
+        if (nc == 1 && n <= slots) break;  // a single round of the quickest workgroups
+        if (nc == 1 || c < least) best = nc, least = c;
     }
     return best;
 }
 
 // Launches pick(columns), the kernel for a column count, where x's planes take
 // `planes` bytes of LDS a column and the staging areas `rest`; cap: workgroups
-// per CU at most.  Planes of over 40 KiB a column stay one by one: a group of
-// them leaves one workgroup of four wavefronts a CU (Q4_K 4096x14336, 6
-// columns: 37 us one by one, 50 in pairs).
-template <class Pick>
+// per CU at most.
+template <int KIND, class Pick>
 int launch_mfma(const char *what, Pick pick, const KqArgs &a, int tiles, int cap, size_t planes, size_t rest, bool sh,
                 hipStream_t s) {
     const size_t red = sh ? kShRed : 0;
-    const int fit = planes > 40 * 1024 ? 1 : static_cast<int>((kLdsMax - rest) / (planes + red));
-    const int nc = kq_columns(a.k, fit, tiles, 2LL * cu_count());
+    const int nc = mfma_columns(a.k, kDecode<KIND>, tiles, cap, planes + red, rest);
     const size_t lds = nc * (planes + red) + rest;
     void (*fn)(KqArgs) = nc == 1 ? pick(std::integral_constant<int, 1>{})
                          : nc == 2 ? pick(std::integral_constant<int, 2>{})
@@ -1631,7 +1670,7 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
         const int nb = a.in_len / 256;
         const size_t planes = static_cast<size_t>(nb) * kQ45Unit, rest = kQ3Waves * 16 * kQ8Seg;
         if (al16 && a.in_len % 256 == 0 && kq_tiling(a.out_len, planes + rest, nb, true) == 1)
-            return launch_mfma("kq8_mfma_kernel", [](auto n) { return kq8_mfma_kernel<decltype(n)::value>; }, a, t16, 4,
+            return launch_mfma<KIND>("kq8_mfma_kernel", [](auto n) { return kq8_mfma_kernel<decltype(n)::value>; }, a, t16, 4,
                                planes, rest, true, s);
     }
     if constexpr (KIND == OURO_KIND_Q6K) {
@@ -1641,9 +1680,9 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
         const int til = kq_tiling(a.out_len, planes + rest, nb / 2, true);
         if (reinterpret_cast<uintptr_t>(a.w) % 4 == 0 && ph && til >= 0) {
             if (til == 1)
-                return launch_mfma("kq6_mfma_kernel", [](auto n) { return kq6_mfma_kernel<true, decltype(n)::value>; }, a,
+                return launch_mfma<KIND>("kq6_mfma_kernel", [](auto n) { return kq6_mfma_kernel<true, decltype(n)::value>; }, a,
                                    t16, 3, planes, rest, true, s);
-            return launch_mfma("kq6_mfma_kernel", [](auto n) { return kq6_mfma_kernel<false, decltype(n)::value>; }, a, t64,
+            return launch_mfma<KIND>("kq6_mfma_kernel", [](auto n) { return kq6_mfma_kernel<false, decltype(n)::value>; }, a, t64,
                                3, planes, rest, false, s);
         }
     }
@@ -1654,10 +1693,10 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
         const int til = kq_tiling(a.out_len, planes + rest, nb, true);
         if (al16 && til >= 0) {
             if (til == 1)
-                return launch_mfma("kq45_mfma_kernel",
+                return launch_mfma<KIND>("kq45_mfma_kernel",
                                    [](auto n) { return kq45_mfma_kernel<KIND, true, decltype(n)::value>; }, a, t16, 4,
                                    planes, rest, true, s);
-            return launch_mfma("kq45_mfma_kernel", [](auto n) { return kq45_mfma_kernel<KIND, false, decltype(n)::value>; },
+            return launch_mfma<KIND>("kq45_mfma_kernel", [](auto n) { return kq45_mfma_kernel<KIND, false, decltype(n)::value>; },
                                a, t64, 4, planes, rest, false, s);
         }
     }
@@ -1669,13 +1708,13 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
             const size_t planes = static_cast<size_t>(nb) * kQ3Unit, rest = kQ3Waves * kQ3Stage;
             const int til = al ? kq_tiling(a.out_len, planes + rest, nb / 2, false) : -1;
             if (til == 1)
-                return launch_mfma("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_STS, decltype(n)::value>; }, a,
+                return launch_mfma<KIND>("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_STS, decltype(n)::value>; }, a,
                                    t16, 4, planes, rest, true, s);
             if (til == 0)
-                return launch_mfma("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_ST, decltype(n)::value>; }, a,
+                return launch_mfma<KIND>("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_ST, decltype(n)::value>; }, a,
                                    t64, 4, planes, rest, false, s);
             if (!al && kq_tiling(a.out_len, planes, nb, false) == 0)  // unstaged: each lane loads its own pieces
-                return launch_mfma("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_ANY, decltype(n)::value>; }, a,
+                return launch_mfma<KIND>("kq3_mfma_kernel", [](auto n) { return kq3_mfma_kernel<Q3K_ANY, decltype(n)::value>; }, a,
                                    t64, 4, planes, 0, false, s);
         }
     }
@@ -1699,17 +1738,22 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
         else if (ph) hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, true, MAXT, NC>), grid, dim3(nt), lds, s, a);
         else hipLaunchKernelGGL((kq_gemv_kernel<KIND, R, false, false, MAXT, NC>), grid, dim3(nt), lds, s, a);
     };
-    constexpr std::integral_constant<int, kRows<KIND>> rows{};
     constexpr std::integral_constant<int, 1> c1{};
+    constexpr std::integral_constant<int, 2> r2{};
     constexpr std::integral_constant<int, 512> t512{};
     // Several columns: four rows a tile where that still gives every workgroup
     // two tiles, else two (three columns of Q6_K, R = 2 / 4: 32768x1792 24.7 /
-    // 21.5, 4096x14336 24.1 / 21.5, 1500x7168 9.7 / 10.8 us).
+    // 21.5, 4096x14336 24.1 / 21.5, 1500x7168 9.7 / 10.8 us); four columns of
+    // Q3_K and Q5_K leave no registers for four rows.
+    const bool tall = (a.out_len + 3) / 4 >= 2 * wgs;
+    auto rows = [](auto cols_c) {
+        constexpr int NC = decltype(cols_c)::value;
+        constexpr bool two = NC == 4 && (KIND == OURO_KIND_Q3K || KIND == OURO_KIND_Q5K);
+        return std::integral_constant<int, NC == 1 ? kRows<KIND> : two ? 2 : 4>{};
+    };
     auto cols = [&](auto cols_c) {
-        // four columns of Q3_K and Q5_K leave no registers for four rows
-        constexpr int R = decltype(cols_c)::value == 4 && (KIND == OURO_KIND_Q3K || KIND == OURO_KIND_Q5K) ? 2 : 4;
-        if ((a.out_len + 3) / 4 >= 2 * wgs) go(std::integral_constant<int, R>{}, t512, cols_c);
-        else go(std::integral_constant<int, 2>{}, t512, cols_c);
+        if (tall || decltype(cols_c)::value == 1) go(rows(cols_c), t512, cols_c);
+        else go(r2, t512, cols_c);
     };
     if (nt > 512) {  // 1024 threads leave no registers for a second column's x
         go(c1, std::integral_constant<int, kMaxThreads>{}, c1);
@@ -1717,13 +1761,18 @@ int launch_kind(KqArgs a, bool al16, hipStream_t s) {
         // a column's sums cost more than the decode it would share (four columns,
         // one by one / grouped: Q6_K 60000x768 58.9 / 89.9, 20000x512 20.9 / 32.2,
         // 60000x3072 121 / 143 us)
-        go(rows, t512, c1);
+        cols(c1);
     } else {
-        switch (kq_columns(a.k, 4, (a.out_len + 1) / 2, cu_count() * std::max(1, 1024 / nt) / 2)) {
-        case 1: go(rows, t512, c1); break;
-        case 2: cols(std::integral_constant<int, 2>{}); break;
-        case 3: cols(std::integral_constant<int, 3>{}); break;
-        default: cols(std::integral_constant<int, 4>{}); break;
+        constexpr std::integral_constant<int, 2> c2{};
+        constexpr std::integral_constant<int, 3> c3{};
+        constexpr std::integral_constant<int, 4> c4{};
+        switch (task_columns(a.k, a.out_len, wgs, [&](int nc) {
+            return nc == 1 ? rows(c1).value : !tall ? 2 : nc == 2 ? rows(c2).value : nc == 3 ? rows(c3).value : rows(c4).value;
+        })) {
+        case 1: cols(c1); break;
+        case 2: cols(c2); break;
+        case 3: cols(c3); break;
+        default: cols(c4); break;
         }
     }
     return check_launch("kq_gemv_kernel");
