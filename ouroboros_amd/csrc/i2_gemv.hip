@@ -621,13 +621,18 @@ int i2_gemm(const uint8_t *w_tiled, size_t out_len, size_t in_len, const float *
 }
 
 // y = W x for one fp32 column in one launch (the product quantises x itself).
-// Each wavefront does that for its 8 rows, some 32 operations per group of
-// four elements and lane: past kFusedGroups tiles * groups the separate launch is cheaper
-// (quantise + product -> fused: 6912x2560 7.7 -> 3.9, 2560x6912 12.8 -> 7.1,
-// 8192x8192 14.8 -> 9.1, 32768x2048, at the line, 8.0 -> 6.9 us).
-constexpr size_t kFusedGroups = 32768;
+// Each wavefront does that for its 8 rows, work that grows with the tiles and
+// with their groups (of 256 elements) and a little more, where the separate
+// launch costs a fixed time: it pays while tiles * (groups + 4) is small (us, quantise and
+// product / fused, cold: 131072x256, 16384 tiles, 7.2 / 6.9 and 196608x256 8.6 / 9.1;
+// 65536x1024 8.3 / 7.0 and 98304x1024 9.6 / 9.6; 32768x2048 8.0 / 6.9 and 49152x2048
+// 9.0 / 8.9; 24576x4096 10.1 / 8.9 and 32768x4096 11.4 / 10.6; small ones 6.6 / 3.7).  Rows of
+// more than 16 groups, whose x a wavefront reads twice, run at one wavefront a
+// SIMD: one round of them is even (8192x5120 7.9 / 8.2, 8192x6912 8.8 / 8.4 and
+// 2560x6912 8.0 / 7.5) and needs no scratch, more lose (13104x5120 9.3 / 11.7).
 bool i2_matvec_f32_pays(size_t out_len, size_t in_len) {
-    return (out_len + kTileRows - 1) / kTileRows * (in_len / 256) <= kFusedGroups;
+    const size_t tiles = (out_len + kTileRows - 1) / kTileRows, groups = in_len / 256;
+    return groups <= 16 ? tiles * (groups + 4) <= 61440 : tiles <= 1024;
 }
 int i2_matvec_f32(const uint8_t *w_tiled, size_t out_len, size_t in_len, const float *w_scale, const float *x, float *y,
                   void *stream) {

@@ -40,10 +40,12 @@ def test_act_quant_rows(gpu, orc, n, bf16, off):
 
 
 @pytest.mark.parametrize("out_len,in_len", [(1, 256), (9, 512), (33, 1024), (70, 2048), (64, 2560), (65, 3072), (40, 4096),
-                                            (31, 5120), (17, 6144), (100, 6912), (8, 8192), (40000, 1024), (70000, 1024),
-                                            (9000, 8192)])
+                                            (31, 5120), (17, 6144), (100, 6912), (8, 8192), (61440, 1024), (61448, 1024),
+                                            (98304, 256), (98305, 256), (8192, 5120), (8193, 5120), (9000, 8192)])
 def test_matvec_rounds_x_itself(gpu, out_len, in_len):
-    """Both sides of the size rule: 32768 tiles of 8 rows times 256-element groups."""
+    """Every row length that a weight takes, and both sides of the size rule:
+    61440 tiles of 8 rows times 256-element groups and four, 1024 tiles from
+    17 groups on."""
     rng = np.random.default_rng(out_len + in_len)
     w = rng.integers(-1, 2, size=(out_len, in_len)).astype(np.int8)
     h = ops.Weight(QuantKind.I2, i2_pack(w), out_len, in_len, w_scale=0.7)
