@@ -652,11 +652,14 @@ int i2_matvec_f32(const uint8_t *w_tiled, size_t out_len, size_t in_len, const f
     return launch_gemv(a, 1, stream, true);
 }
 
-// act_quant4_kernel for rows of n elements, or the element loop.
+// act_quant4_kernel for rows of n elements, or the element loop: beyond its
+// registers, off its alignment, and for rows that leave three quarters of the
+// workgroup idle (rows of 64, 20000 of them 12.9 against 14.4 us; 10000 of 256
+// 8.8 / 8.3).
 template <typename T>
 void launch_act_quant(const T *x, size_t rows, size_t n, int8_t *xq, float *act_scale, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(rows)), block(256);
-    const bool four = n % 4 == 0 && n <= 4 * 256 * kQuantRegs && reinterpret_cast<uintptr_t>(xq) % 4 == 0 &&
+    const bool four = n % 4 == 0 && n >= 256 && n <= 4 * 256 * kQuantRegs && reinterpret_cast<uintptr_t>(xq) % 4 == 0 &&
                       reinterpret_cast<uintptr_t>(x) % (sizeof(T) == 2 ? 8 : 4) == 0;
     const int m = static_cast<int>(n);
     if (!four) hipLaunchKernelGGL(act_quant_kernel<T>, grid, block, 0, s, x, static_cast<long long>(n), xq, act_scale);

@@ -1,7 +1,7 @@
 """Quantisation of activations ahead of a ternary product: whole-integer and
 bit-exact results, whichever kernel runs.  The row kernel with 4-element loads
-(rows of whole groups up to 8192) at its register-count edges, the element
-loop beyond and on odd lengths or addresses; and a resident weight's matvec,
+(rows of whole groups, 256 to 8192) at its register-count edges, the element
+loop on either side and on odd lengths or addresses; and a resident weight's matvec,
 which rounds x inside the product below a size, against the two calls
 ouro_act_quant_i8 and ouro_gemm_i2 at every row length that a weight takes."""
 import numpy as np
@@ -22,7 +22,7 @@ def inputs(rng, rows, n):
     return x
 
 
-@pytest.mark.parametrize("n", [1, 4, 7, 1020, 1024, 2048, 2052, 4096, 4100, 6912, 8192, 8196, 4098])
+@pytest.mark.parametrize("n", [1, 4, 7, 252, 256, 1020, 1024, 2048, 2052, 4096, 4100, 6912, 8192, 8196, 4098])
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("off", [0, 1])
 def test_act_quant_rows(gpu, orc, n, bf16, off):
