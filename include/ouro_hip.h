@@ -275,7 +275,11 @@ int ouro_gemm_i2_mfma(const uint8_t *w_mfma, size_t out_len, size_t in_len,
  *   weight handle keeps these calls allocation-free).
  * Floating-point sums are not in the reference's order; results agree to
  * float32 rounding (the reference's own fused-vs-scalar bar is rel 1e-5,
- * ops.rs:800-838). */
+ * ops.rs:800-838).  A column of ouro_matmul_q has the bits of ouro_matvec_q of
+ * it on the block-quantised and 2-bit kinds; on dense rows one column, two to
+ * four, and more are summed in three orders, which agree to float32 rounding
+ * only (a column's bits do not depend on how many beyond that), and the
+ * number of rows may change the order too. */
 int ouro_matvec_q(const void *payload, int kind, size_t out_len,
                   size_t in_len, const float *x, float *y, void *stream);
 /* matmul_q (ops.rs:219-230): x row-major [k][in_len], y column-major

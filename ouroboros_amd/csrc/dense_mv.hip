@@ -308,10 +308,10 @@ int launch_cols(const DenseArgs &a, bool al, hipStream_t s) {
     constexpr int NC = kCols<WIDE>;
     const dim3 grid((a.out_len - 1) / kDenseRows + 1, (a.k - 1) / NC + 1);
     const int steps = (a.in_len - 1) / kStep<KIND, WIDE> + 1;
-    // about 16 wavefronts a CU over the grid, the steps spread evenly over a
-    // workgroup's wavefronts
-    const long long wgs = static_cast<long long>(grid.x) * grid.y;
-    int nw = static_cast<int>(std::min<long long>(std::min(kMaxWaves<WIDE>, steps), (4096 + wgs - 1) / wgs));
+    // about 16 wavefronts a CU over the rows, the steps spread evenly over a
+    // workgroup's wavefronts; not by the column groups, so that a column's sum
+    // is the same in any number of them
+    int nw = static_cast<int>(std::min<unsigned>(std::min(kMaxWaves<WIDE>, steps), (4095 + grid.x) / grid.x));
     const int per = (steps + nw - 1) / nw;
     nw = (steps + per - 1) / per;
     const size_t lds = static_cast<size_t>(nw) * std::min(NC, a.k) * kXPitch<KIND, WIDE> * sizeof(float);

@@ -70,3 +70,18 @@ def test_dense_non_finite_and_tiny(gpu, k):
     tiny = np.full((out_len, in_len), 1e-20, np.float32)
     got = run(tiny.view(np.uint8).reshape(-1), QuantKind.F32, out_len, in_len, np.full((k, in_len), 1e-20, np.float32))
     assert np.allclose(got, in_len * 1e-40, rtol=1e-3, atol=0)
+
+
+@pytest.mark.parametrize("kind", [QuantKind.F32, QuantKind.BF16], ids=lambda k: k.name)
+@pytest.mark.parametrize("out_len,in_len", [(4096, 2050), (600, 3001), (33, 129)])
+def test_dense_column_in_any_number(gpu, kind, out_len, in_len):
+    """A column has the same bits among two, three or four columns, and the
+    same among any larger number (one column, these and those are summed in
+    three orders)."""
+    rng = np.random.default_rng(out_len)
+    _, payload = weights(rng, kind, out_len, in_len)
+    x = rng.standard_normal((40, in_len)).astype(np.float32)
+    for few, many in (((2, 3), 4), ((5, 16, 17, 33), 40)):
+        whole = run(payload, kind, out_len, in_len, x[:many])
+        for k in few:
+            assert np.array_equal(run(payload, kind, out_len, in_len, x[:k]), whole[:k]), k
