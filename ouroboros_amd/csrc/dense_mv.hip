@@ -315,8 +315,8 @@ int launch_cols(const DenseArgs &a, bool al, hipStream_t s) {
     const int per = (steps + nw - 1) / nw;
     nw = (steps + per - 1) / per;
     const size_t lds = static_cast<size_t>(nw) * std::min(NC, a.k) * kXPitch<KIND, WIDE> * sizeof(float);
-    if (al) hipLaunchKernelGGL((dense_mv_kernel<KIND, WIDE, true>), grid, dim3(64 * nw), lds, s, a);
-    else hipLaunchKernelGGL((dense_mv_kernel<KIND, WIDE, false>), grid, dim3(64 * nw), lds, s, a);
+    const auto fn = al ? dense_mv_kernel<KIND, WIDE, true> : dense_mv_kernel<KIND, WIDE, KIND == OURO_KIND_F32>;
+    hipLaunchKernelGGL(fn, grid, dim3(64 * nw), lds, s, a);
     return check_launch("dense_mv_kernel");
 }
 
@@ -327,14 +327,14 @@ int launch_vec(const DenseArgs &a, bool al, hipStream_t s) {
     int nw = static_cast<int>(std::min<unsigned>(std::min(kVecWaves, steps), (4096 + wgs - 1) / wgs));
     const int per = (steps + nw - 1) / nw;
     nw = (steps + per - 1) / per;
-    if (al) hipLaunchKernelGGL((dense_vec_kernel<KIND, R, true>), dim3(wgs), dim3(64 * nw), 0, s, a);
-    else hipLaunchKernelGGL((dense_vec_kernel<KIND, R, false>), dim3(wgs), dim3(64 * nw), 0, s, a);
+    const auto fn = al ? dense_vec_kernel<KIND, R, true> : dense_vec_kernel<KIND, R, KIND == OURO_KIND_F32>;
+    hipLaunchKernelGGL(fn, dim3(wgs), dim3(64 * nw), 0, s, a);
     return check_launch("dense_vec_kernel");
 }
 
 template <int KIND>
 int launch_kind(const DenseArgs &a, hipStream_t s) {
-    // every row on a dword
+    // every row on a dword (fp32 always)
     const bool al = KIND == OURO_KIND_F32 || (a.in_len % 2 == 0 && reinterpret_cast<uintptr_t>(a.w) % 4 == 0);
     if (a.k == 1) return a.out_len >= 4096 ? launch_vec<KIND, 4>(a, al, s) : launch_vec<KIND, 1>(a, al, s);
     return a.k > kCols<false> ? launch_cols<KIND, true>(a, al, s) : launch_cols<KIND, false>(a, al, s);
