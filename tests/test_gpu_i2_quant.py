@@ -24,17 +24,20 @@ def inputs(rng, rows, n):
 
 @pytest.mark.parametrize("n", [1, 4, 7, 252, 256, 1020, 1024, 2048, 2052, 4096, 4100, 6912, 8192, 8196, 4098])
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("off", [0, 1])
-def test_act_quant_rows(gpu, orc, n, bf16, off):
+@pytest.mark.parametrize("off", [0, 1])  # bytes that xq lies past its boundary
+@pytest.mark.parametrize("x_off", [0, 1, 2])  # elements that x lies past a 16-byte boundary
+def test_act_quant_rows(gpu, orc, n, bf16, off, x_off):
     rows = 5
     x = inputs(np.random.default_rng(n), rows, n)
     bits = f32_to_bf16_bits(x)
     if bf16:
         x = bf16_bits_to_f32(bits).reshape(rows, n)
     want_q, want_s = orc.act_quant_i8(x)
-    xd = DeviceBuffer.from_host(bits if bf16 else x)
+    src = (bits if bf16 else x).reshape(-1)
+    xd = DeviceBuffer.from_host(np.concatenate([np.zeros(x_off, src.dtype), src]))
+    xp = xd.ptr + x_off * src.itemsize
     q, s = DeviceBuffer((rows * n + 16,), np.int8), DeviceBuffer((rows,), np.float32)
-    call("ouro_act_quant_i8", xd.ptr, DT_BF16 if bf16 else DT_F32, rows, n, q.ptr + off, s.ptr, None)
+    call("ouro_act_quant_i8", xp, DT_BF16 if bf16 else DT_F32, rows, n, q.ptr + off, s.ptr, None)
     assert np.array_equal(q.download()[off:off + rows * n].reshape(rows, n), want_q)
     assert np.array_equal(s.download().view(np.uint32), want_s.view(np.uint32))
 
@@ -55,12 +58,13 @@ def test_matvec_rounds_x_itself(gpu, out_len, in_len):
     payload = _lib.lib().ouro_weight_payload(h.handle)
     scale = payload + _lib.lib().ouro_i2_tiled_bytes(out_len, in_len)
     rows = np.concatenate([x, inputs(rng, 2, in_len)[1:]])
-    for row in rows:
-        xd = DeviceBuffer.from_host(row)
+    for x_off, row in enumerate(rows):  # the product reads x at any 4-byte boundary
+        xd = DeviceBuffer.from_host(np.concatenate([np.zeros(x_off, np.float32), row]))
+        xp = xd.ptr + 4 * x_off
         q, s = DeviceBuffer((in_len,), np.int8), DeviceBuffer((1,), np.float32)
         y, y2 = DeviceBuffer((out_len,), np.float32), DeviceBuffer((out_len,), np.float32)
-        call("ouro_weight_matvec", h.handle, xd.ptr, y.ptr, None)
-        call("ouro_act_quant_i8", xd.ptr, DT_F32, 1, in_len, q.ptr, s.ptr, None)
+        call("ouro_weight_matvec", h.handle, xp, y.ptr, None)
+        call("ouro_act_quant_i8", xp, DT_F32, 1, in_len, q.ptr, s.ptr, None)
         call("ouro_gemm_i2", payload, out_len, in_len, scale, q.ptr, s.ptr, 1, y2.ptr, None, None)
         assert np.array_equal(y.download().view(np.uint32), y2.download().view(np.uint32))
 
