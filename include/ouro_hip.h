@@ -291,9 +291,9 @@ int ouro_matmul_q(const void *payload, int kind, size_t out_len,
  * hipMalloc (code under HIP graph capture, tight serving loops, harnesses
  * that forbid allocation).  No counterpart in the reference.  It uses a
  * static per-device scratch array of 16 MiB that each device holds until
- * the process ends.  For the 2-bit kinds (OURO_KIND_I2_S, OURO_KIND_I2) x
- * is quantised into its first 32 KiB + 256 B, so in_len <= 32768
- * (OURO_ERR_SHAPE beyond).  TL1 and TQ1_0 payloads of 8192 rows or more
+ * the process ends.  For the 2-bit kinds (OURO_KIND_I2_S, and OURO_KIND_I2
+ * where the product does not quantise x itself) x is quantised into its
+ * first 32 KiB + 256 B; in_len <= 32768 (OURO_ERR_SHAPE beyond).  TL1 and TQ1_0 payloads of 8192 rows or more
  * keep the table-lookup kernels' per-block partial sums there when they fit
  * (TL1: ceil(in_len/512) * out_len floats, TQ1_0: in_len/512 * out_len,
  * at most 16 MiB: the 248320x5120 lm_head takes 9.9 MB); larger ones run

@@ -2,8 +2,12 @@
 // 131-154, 600-623) for one or several columns.
 //
 // Weights widen exactly to fp32 and x stays fp32, so the products and sums
-// are those of fp32 arithmetic for every kind, in chains of at most a few
-// products per partial sum.  Rows may start at any element.
+// are those of fp32 arithmetic for every kind.  Chains: one column, one per
+// element of a piece over a wavefront's steps (56 products at most, F32 rows
+// of 14336 elements on one wavefront), then trees; several, eight a step of
+// up to 8 products, a tree over them, then one over the wavefront's steps.
+// Rows may start at any element.  One column, two to four, and more are three
+// summation orders; within each a column does not depend on the others.
 //
 // One column: dense_vec_kernel, 16-byte loads on the vector ALU.  Several:
 // dense_mv_kernel on the fp32 matrix cores, one pass over the payload for up
@@ -27,7 +31,8 @@
 // vector products that stood here: bf16 8192x2560, 1 / 4 / 6 columns 16.0 /
 // 49.5 / 81 -> 8.4 / 9.8 / 11.4 us (42 MB: 5.0 / 4.3 / 3.7 TB/s), 4096x4096
 // with 16 columns 131 -> 11.2, 32768x2047 with 16 (odd rows) 527 -> 43 us;
-// fp32 4096x14336, one column, 77.5 -> 32.4 us.
+// fp32 4096x14336, one column, 77.5 -> 32.4 us.  Slower only on rows that do not
+// fill a step: 100x100, 2 to 4 columns, 3.1 -> 4.1 us.
 #include "common.hpp"
 
 #include <algorithm>

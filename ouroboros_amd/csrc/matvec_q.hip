@@ -306,7 +306,8 @@ int matmul_q(const void *payload, int kind, size_t out_len, size_t in_len, const
 //
 // Callers that cannot allocate (code under HIP graph capture, tight serving
 // loops) get ouro_matvec_q_noalloc: its 2-bit kinds quantise x into this
-// file-scope device array, and its TL1 / TQ1_0 lookup GEMVs keep their
+// file-scope device array (tiled I2 past i2_matvec_f32_pays and in place only:
+// else the product rounds x itself), and its TL1 / TQ1_0 lookup GEMVs keep their
 // per-block partial sums there, instead of the library workspace.  Each
 // device holds its own copy until the process ends; its address on a device
 // comes from hipGetSymbolAddress (the array's name is not a device address
