@@ -250,11 +250,13 @@ def test_kquant_shape_errors(gpu):
 @pytest.mark.parametrize("kind", KINDS, ids=lambda k: k.name)
 @pytest.mark.parametrize("out_len,in_len,offset", [(37, 768, 0), (97, 14336, 0), (300, 20480, 0), (2100, 768, 0),
                                                    (2100, 1024, 2), (4100, 4096, 0), (8200, 8192, 0), (16399, 1536, 4),
-                                                   (16399, 10752, 0)])
+                                                   (16399, 10752, 0), (8200, 13568, 0), (3000, 8192, 0),
+                                                   (3001, 1536, 1), (600, 3072, 1), (200, 16384, 1)])
 def test_kquant_column_groups(gpu, kind, out_len, in_len, offset):
     """Columns are taken 1 to 4 at a time, by the task kernel and by each
     tiling of the matrix-core kernels (planes of several columns past 64 KiB
-    of LDS among them); whatever the group, each column is the matvec of that
+    of LDS, up to the 160 of a CU, among them, and rows that share a workgroup,
+    one column at a time); whatever the group, each column is the matvec of that
     column bit for bit (which the tests above hold to the oracle), with a
     ragged last group too."""
     rng = np.random.default_rng(out_len + in_len + offset)
